@@ -358,7 +358,7 @@ typedef struct sas_spec_state {
  * round is ignored), `st` the sequences' persistent state. */
 int sas_spec_step(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *st, void *stream);
 
-/* ---- the LM head with the sampling step fused into its epilogue ----
+/* ---- the LM head with the sampling step fused behind it ----
  *
  * Replaces the decode head's final projection and the topk pass that reads
  * its logits: lib/webgpu-llm/model.js:466-471 (Qwen: rms -> lm per
@@ -373,9 +373,9 @@ int sas_spec_step(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *
  * partial sums, partial g a fused multiply-add chain from 0 over
  * k = 64 c + 8 g + j (c ascending, then j = 0 .. 7), added as
  * ((p0 + p1) + (p2 + p3)) + ((p4 + p5) + (p6 + p7)).  The logits
- * are consumed on chip: no [rows][vocab] array is written unless
- * out_logits asks for it.  Then the sas_sample semantics over them
- * (softcap, mask, penalties, top-k / top-p, draw). */
+ * go to out_logits when it is set, else to the handle's scratch.  Then the
+ * sas_sample semantics over them (softcap, mask, penalties, top-k / top-p,
+ * draw). */
 #define SAS_LMH_MAX_ROWS 4        /* rows per call: decode (1) and verify rounds (3) */
 #define SAS_LMH_MAX_LDS_FLOATS 12288  /* rows * dim: the hidden states staged on chip */
 #define SAS_LMH_MAX_VOCAB 262144      /* vocabularies of the fused head */

@@ -26,6 +26,8 @@ struct sas_sampler {
   size_t vscratch_cap = 0;
   void *pad = nullptr;        // rows of fewer than 4 logits, padded to 4
   size_t pad_cap = 0;
+  void *logits = nullptr;     // the LM head's logits (sas_lm_head_sample without out_logits)
+  size_t logits_cap = 0;
   void *hb = nullptr;         // long histories bucketed by part
   size_t hb_cap = 0;
   int cus = 0;                 // compute units of the device
@@ -193,9 +195,10 @@ struct SpecDraw {
 };
 
 // sas_sample, sas_sample_step (st) and the sampling of sas_spec_exact (sp):
-// one checked descriptor's launches.
+// one checked descriptor's launches.  bucket: long histories may be
+// bucketed first (not behind the LM head, whose scratch holds no buckets).
 int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char *who, void *stream,
-              const SpecDraw *sp = nullptr) {
+              const SpecDraw *sp = nullptr, bool bucket = true) {
   if (int rc = set_device(s)) return rc;
   // at least two blocks per CU: small batches take shorter parts
   int parts = 0, span = 0;
@@ -241,7 +244,7 @@ int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char 
   const int hrows = sp && sp->group > 1 ? r->rows / sp->group : r->rows;
   const bool ring = a.ring != nullptr;
   const int64_t hist_ids = ring ? (int64_t)hrows * a.ring_len : (r->hist_ids ? r->hist_count : 0);
-  if (hist_ids >= sas::kBucketMinIds * hrows && hist_ids > 0) {
+  if (bucket && hist_ids >= sas::kBucketMinIds * hrows && hist_ids > 0) {
     const size_t ids_bytes = ((size_t)hist_ids * 4 + 255) & ~size_t(255);
     if (int rc = grow(s, &s->hb, &s->hb_cap, hb_bytes(hist_ids, hrows, parts), stream, who)) return rc;
     a.hb_ids = reinterpret_cast<uint32_t *>(s->hb);
@@ -260,6 +263,20 @@ int64_t head_row_bytes(int32_t format, int32_t dim) {
     case SAS_HEAD_Q6_K: return (int64_t)dim / 256 * 210;
     default: return 0;
   }
+}
+
+// Floats between the rows of the head's logits in the handle's scratch.
+int64_t lmh_logits_stride(int32_t vocab) { return ((int64_t)vocab + 3) & ~int64_t(3); }
+
+// The scratch of the LM head's calls of at most `rows` rows at `vocab`: the
+// logits and the sampling step's records (parts hold 1,024 ids or more) and
+// padded rows.
+int ensure_lmh_scratch(sas_sampler *s, int rows, int vocab, void *stream, const char *who) {
+  const int parts = std::min(sas::kMaxParts, (vocab + 1023) / 1024);
+  if (int rc = ensure_sample_scratch(s, rows, parts, stream, who)) return rc;
+  if (vocab < 4)
+    if (int rc = grow(s, &s->pad, &s->pad_cap, (size_t)rows * 16, stream, who)) return rc;
+  return grow(s, &s->logits, &s->logits_cap, (size_t)rows * lmh_logits_stride(vocab) * sizeof(float), stream, who);
 }
 
 // sas_lm_head_sample and sas_lm_head_sample_step (st).
@@ -305,30 +322,26 @@ int lm_head_on(sas_sampler *s, const sas_lm_head *h, const sas_rows *r, const sa
   if (reinterpret_cast<uintptr_t>(h->hidden) % 4 != 0)
     return fail(s, SAS_ERR_INVALID, w + ": hidden must be 4-byte aligned");
   if (int rc = set_device(s)) return rc;
-  if (int rc = grow(s, &s->recs, &s->recs_cap, sas::lmh_scratch_bytes(r->rows, r->vocab), stream, who)) return rc;
+  // all scratch before the first launch (a capture that lacks some records nothing)
+  if (int rc = ensure_lmh_scratch(s, r->rows, r->vocab, stream, who)) return rc;
   sas::LmhArgs a{};
-  fill_args(r, nullptr, 0, 1, sas::kLmhSpan, s->recs, &a.s);
-  sas::lmh_layout(&a, s->recs);
-  if (st) {
-    a.s.st_state = st->state;
-    a.s.st_sampled = st->sampled;
-    a.s.st_max_steps = st->sampled ? st->max_steps : 0;
-    a.s.st_next = st->next_tokens;
-    a.s.ring = st->ring;
-    a.s.ring_len = st->ring ? st->ring_len : 0;
-    a.s.stop_ids = st->stop_ids;
-    a.s.seeds = st->seeds;
-  }
   a.hidden = h->hidden;
   a.hidden_stride = h->hidden_stride;
   a.weight = h->weight;
   a.weight_stride = h->weight_stride;
+  a.logits = h->out_logits ? h->out_logits : reinterpret_cast<float *>(s->logits);
+  a.logits_stride = h->out_logits ? (int64_t)r->vocab : lmh_logits_stride(r->vocab);
   a.format = h->format;
   a.dim = h->dim;
-  a.out_logits = h->out_logits;
-  hipError_t e = sas::launch_lm_head_sample(a, any_softcap(r), pick_stream(s, stream));
+  a.vocab = r->vocab;
+  a.rows = r->rows;
+  a.blocks = sas::lmh_blocks(r->vocab, s->cus);
+  hipError_t e = sas::launch_lm_head(a, pick_stream(s, stream));
   if (e != hipSuccess) return hip_fail(s, e, (w + " launch").c_str());
-  return SAS_OK;
+  sas_rows lr = *r;
+  lr.logits = a.logits;
+  lr.logits_stride = a.logits_stride;
+  return sample_on(s, &lr, st, who, stream, nullptr, false);
 }
 
 }  // namespace
@@ -374,6 +387,7 @@ void sas_destroy(sas_sampler *s) {
   for (void *p : s->retired) (void)hipFree(p);
   if (s->recs) (void)hipFree(s->recs);
   if (s->hb) (void)hipFree(s->hb);
+  if (s->logits) (void)hipFree(s->logits);
   if (s->vscratch) (void)hipFree(s->vscratch);
   if (s->pad) (void)hipFree(s->pad);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -406,9 +420,9 @@ int sas_reserve_for(sas_sampler *s, const sas_reserve_desc *d) {
   // the most parts any batch of <= rows rows may pick (a single row)
   int parts = 0, span = 0;
   sas::choose_parts(1, d->vocab, 2 * s->cus, &parts, &span);
-  size_t recs = sas::sample_rec_bytes(d->rows, parts);
-  if (d->lm_head_rows > 0) recs = std::max(recs, sas::lmh_scratch_bytes(d->lm_head_rows, d->vocab));
-  if (int rc = grow(s, &s->recs, &s->recs_cap, recs, nullptr, who)) return rc;
+  if (int rc = ensure_sample_scratch(s, d->rows, parts, nullptr, who)) return rc;
+  if (d->lm_head_rows > 0)
+    if (int rc = ensure_lmh_scratch(s, d->lm_head_rows, d->vocab, nullptr, who)) return rc;
   if (d->vocab < 4 && d->rows > 0)
     if (int rc = grow(s, &s->pad, &s->pad_cap, (size_t)d->rows * 16, nullptr, who)) return rc;
   if (d->hist_ids >= sas::kBucketMinIds && d->rows > 0)

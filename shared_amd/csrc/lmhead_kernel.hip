@@ -1,298 +1,39 @@
-// lmhead_kernel.hip - the LM head with the sampling step's parts pass fused
-// into its epilogue (gfx950).
+// lmhead_kernel.hip - the LM head's logits for the decode head with the
+// sampling step fused behind it (gfx950).
 //
 // The decode head of the reference is a projection of the final-normed
 // hidden state onto every vocabulary row, then a topk pass that reads the
 // logits back (lib/webgpu-llm/model.js:466-471, gemma-model.js:786-799).
-// Here the logits never leave the chip: the block that computes a part's
-// logits also masks, penalizes and bounds them and writes only the part's
-// candidate records, in the records format of the sampling kernels.
-//
-// lmh_parts_kernel: grid = parts (kLmhSpan ids each), 256 threads, every
-// row of the call (<= SAS_LMH_MAX_ROWS).  The rows' hidden states are staged
-// once in LDS.  Eight lanes share one id: lane g of the group sums the
-// hidden indices 64 c + 8 g .. + 7 (c ascending) as one f32 fused
-// multiply-add chain, so each load of the group is a whole 128-byte line of
-// the weight row; the eight partial sums then add in one fixed tree.  That
-// order is the one the host oracle follows.  The bf16 weight widens exactly
-// to f32 (bits << 16, ggml/kernels.js:31-33), so each product is the
-// reference's f32 product.
-// The epilogue, per row: softcap, mask, history membership, the part's
-// bound (every wave's j-th largest lane maximum, the smallest of the four:
-// 4 j >= k values reach it), the values at or above it as records, the
-// members' penalized doubles as member records, the part's info word.
-//
-// lmh_group_kernel: one block per (row, kLmhGroup consecutive parts) keeps
-// the records at or above the group's k-th largest key (at or above the
-// largest of the parts' bounds: that part alone holds k values above it)
-// and writes them as one part of the merge kernel, which then draws as for
+// lmh_logits_kernel streams the head once for every row of the call
+// (<= SAS_LMH_MAX_ROWS) and writes f32 logits (1 MB per row at 262,144 ids,
+// against 1.3 GB of bf16 head); the sampling kernels then take them as for
 // sas_sample.
+//
+// Eight lanes share one id: lane g of the group sums the hidden indices
+// 64 c + 8 g .. + 7 (c ascending) as one f32 fused multiply-add chain, so
+// each load of the group is a whole 128-byte line of the weight row; the
+// eight partial sums then add in one fixed tree.  That order is the one the
+// host oracle follows.  The bf16 weight widens exactly to f32 (bits << 16,
+// ggml/kernels.js:31-33), so each product is the reference's f32 product.
+//
+// Bound by HBM (2 R flops per 2-byte weight): every wave walks the
+// vocabulary in groups of 8 ids, wave w of the grid taking groups w,
+// w + waves, ..., so that whatever the vocabulary every CU streams until the
+// end.  (Blocks of 512 consecutive ids with the sampling pass over them in
+// the same block left CUs idle below 131,072 ids, and folding their records
+// took a launch of its own.  A whole call before -> now: Q4_0 32,000 x
+// 4,096, one row, 91.7 -> 31.2 us; Q6_K 248,320 x 2,560, three rows, 129.2
+// -> 117.9 us; bf16 262,144 x 2,560, one row, 217.1 -> 215.0 us, 6.7 TB/s
+// in this kernel.)
 #include "sas_device.h"
 #include "sas_launch.h"
 
 namespace sas {
 
-constexpr int kLmhIds = kLmhSpan / kThreads;  // ids per lane
-static_assert(kLmhIds == 2, "a lane owns two ids of its part");
-constexpr int kLmhStep = 64;                   // hidden values per load step: 128 bytes of a weight row
-constexpr int kLmhHash = 512;                  // (id, count) hash slots of a part's history members
-constexpr uint32_t kLmhEmpty = 0xFFFFFFFFu;
-
-// The epilogue's tables, one set per row of the call: the rows are
-// selected together, so each barrier serves all of them.
-template <int R>
-struct LmhLds {
-  uint32_t hkey[R][kLmhHash];
-  uint32_t hcnt[R][kLmhHash];
-  uint32_t hbits[R][kLmhSpan / 32];  // history membership of the part's ids
-  uint32_t thr[R][kWaves];           // each wave's bound key
-  uint32_t nw[R][kWaves];            // each wave's plain records
-  uint32_t nmem[R];                  // members kept at or above the bound
-  uint32_t nmw[R];                   // member records written
-  uint32_t hover[R];                 // some history id did not fit in the hash
-  uint32_t nx, slow;                 // an exact selection's plain records, and whether one ran
-  uint32_t hist[256];                // block_select96
-  uint32_t sel[4];
-};
-
-__device__ __forceinline__ uint32_t lmh_slot(uint32_t id) { return (id * 2654435761u) >> 23; }
-static_assert(kLmhHash == 512, "lmh_slot yields 9 bits");
+constexpr int kLmhStep = 64;  // hidden values per load step: 128 bytes of a weight row
 
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-
-// What the epilogue of one row reads from memory, loaded when the block
-// starts so that no round trip waits after the dot products: the row's
-// history range, its first 2 x 256 history ids, the mask word of this
-// lane's two ids.
-struct LmhPre {
-  int h0, h1;
-  const uint32_t *ids;  // the history: hist_ids, or the row's ring slots
-  uint32_t hid[2];
-  uint32_t mword;
-};
-
-// The history range and the mask word (no load depends on another)...
-__device__ __forceinline__ void lmh_prefetch_range(const SampleArgs &a, int row, int id0, LmhPre &q) {
-  q.h0 = 0;
-  q.h1 = 0;
-  q.ids = a.hist_ids;
-  if (a.ring) {
-    // a decode step's penalty ring: its first min(count, ring_len) slots
-    const uint32_t *rg = a.ring + (int64_t)row * (a.ring_len + 1);
-    q.ids = rg + 1;
-    q.h1 = (int)min(rg[0], (uint32_t)a.ring_len);
-  } else if (a.hist_ids) {
-    const int64_t o0 = min(max((int64_t)a.hist_offsets[row], (int64_t)0), a.hist_count);
-    const int64_t o1 = min(max((int64_t)a.hist_offsets[row + 1], o0), min(a.hist_count, o0 + SAS_MAX_HISTORY));
-    q.h0 = (int)o0;
-    q.h1 = (int)o1;
-  }
-  // id0 is even: both ids share one mask word
-  q.mword = a.mask && id0 < a.vocab ? a.mask[(int64_t)row * a.mask_stride + (id0 >> 5)] : ~0u;
-}
-
-// ... then the first history ids, once the range is known.
-__device__ __forceinline__ void lmh_prefetch_ids(LmhPre &q) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int i = q.h0 + j * kThreads + (int)threadIdx.x;
-    q.hid[j] = i < q.h1 ? q.ids[i] : kLmhEmpty;
-  }
-}
-
-// The part's selection for every row of the call: values v[r][0..1] of ids
-// id0, id0 + 1 (raw logits), each row's parameters and history; writes each
-// row's records and info word.  A member is penalized by the lane that holds
-// it (its count from the row's hash) and kept when it reaches the bound,
-// which comes from the plain values only.
-template <int R>
-__device__ __forceinline__ void lmh_select_rows(const LmhArgs &L, LmhLds<R> &S, int part, const float (&v_in)[R][2],
-                                                int id0, const LmhPre (&pf)[R]) {
-  const SampleArgs &a = L.s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int vocab = a.vocab;
-  const int base = part * kLmhSpan;
-  const int nids = min(kLmhSpan, vocab - base);
-  // ---- history: each row's ids inside the part, in a bitmap and a hash ----
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    for (int s2 = tid; s2 < kLmhHash; s2 += kThreads) {
-      S.hkey[r][s2] = kLmhEmpty;
-      S.hcnt[r][s2] = 0u;
-    }
-    if (tid < kLmhSpan / 32) S.hbits[r][tid] = 0u;
-    if (tid == 0) {
-      S.nmem[r] = 0u;
-      S.nmw[r] = 0u;
-      S.hover[r] = 0u;
-    }
-  }
-  __syncthreads();
-  auto insert = [&](int r, uint32_t id) __attribute__((always_inline)) {
-    const uint32_t off = id - (uint32_t)base;
-    if (off >= (uint32_t)nids) return;
-    atomicOr(&S.hbits[r][off >> 5], 1u << (off & 31u));
-    uint32_t sl = lmh_slot(id);
-    int probe = 0;
-    for (; probe < kLmhHash; ++probe) {
-      const uint32_t old = atomicCAS(&S.hkey[r][sl], kLmhEmpty, id);
-      if (old == kLmhEmpty || old == id) {
-        atomicAdd(&S.hcnt[r][sl], 1u);
-        break;
-      }
-      sl = (sl + 1u) & (uint32_t)(kLmhHash - 1);
-    }
-    if (probe == kLmhHash) S.hover[r] = 1u;
-  };
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    // the first 2 x 256 ids came with the block's first loads (kLmhEmpty past
-    // the range: never inside the part)
-    insert(r, pf[r].hid[0]);
-    insert(r, pf[r].hid[1]);
-    for (int i = pf[r].h0 + 2 * kThreads + tid; i < pf[r].h1; i += kThreads) insert(r, pf[r].ids[i]);
-  }
-  __syncthreads();
-  auto hcount = [&](int r, uint32_t id) -> uint32_t {
-    uint32_t sl = lmh_slot(id);
-    for (int probe = 0; probe < kLmhHash; ++probe) {
-      const uint32_t kk = S.hkey[r][sl];
-      if (kk == id) return S.hcnt[r][sl];
-      if (kk == kLmhEmpty) break;
-      sl = (sl + 1u) & (uint32_t)(kLmhHash - 1);
-    }
-    uint32_t c = 0u;
-    if (S.hover[r])
-      for (int i = pf[r].h0; i < pf[r].h1; ++i) c += pf[r].ids[i] == id ? 1u : 0u;
-    return c;
-  };
-  // ---- values: softcap, mask, membership; members penalized here; the bound ----
-  sas_params p[R];
-  int kr[R];
-  float pv[R][2];   // plain candidates (NaN: none)
-  bool mem[R][2];   // allowed history members
-  double mv[R][2];  // their penalized values
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    p[r] = a.params;
-    if (a.row_params) p[r] = load_row_params(a.row_params + r);
-    kr[r] = !(p[r].temperature > 0.0) ? 1 : min(max(p[r].top_k, 1), SAS_MAX_TOP_K);
-    const uint32_t *mrow = a.mask ? a.mask + (int64_t)r * a.mask_stride : nullptr;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int id = id0 + j;
-      float x = v_in[r][j];
-      if (p[r].softcap > 0.0f) x = softcap_f32(x, p[r].softcap);
-      bool ok = id < vocab && x == x;
-      if (ok && mrow) ok = ((pf[r].mword >> (id & 31)) & 1u) != 0u;
-      const uint32_t off = (uint32_t)(id - base);
-      const bool hm = ok && off < (uint32_t)nids && ((S.hbits[r][off >> 5] >> (off & 31u)) & 1u) != 0u;
-      mem[r][j] = hm;
-      pv[r][j] = ok && !hm ? x : qnan();
-      mv[r][j] = hm ? penalize((double)x, hcount(r, (uint32_t)id), p[r]) : 0.0;
-    }
-    const float m = fmaxf(pv[r][0], pv[r][1]);
-    const uint32_t tw = wave_jth_largest_key16(okey(m), (kr[r] + kWaves - 1) / kWaves);
-    if (lane == 0) S.thr[r][wave] = tw;
-  }
-  __syncthreads();
-  // ---- plain records: each wave's after the waves before it; members kept ----
-  uint32_t tkey[R], pre[R];
-  float tf[R];
-  bool k0[R], k1[R], m0[R], m1[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    tkey[r] = min(min(S.thr[r][0], S.thr[r][1]), min(S.thr[r][2], S.thr[r][3]));
-    tf[r] = tkey[r] > 0x007FFFFFu ? fkey(tkey[r]) : -__builtin_inff();
-    k0[r] = pv[r][0] >= tf[r];  // NaN never passes
-    k1[r] = pv[r][1] >= tf[r];
-    const uint32_t c = (k0[r] ? 1u : 0u) + (k1[r] ? 1u : 0u);
-    const uint64_t b0 = __ballot(c & 1u), b1 = __ballot((c >> 1) & 1u);
-    pre[r] = lanes_below(b0) + 2u * lanes_below(b1);
-    if (lane == 0) S.nw[r][wave] = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1);
-    m0[r] = mem[r][0] && mv[r][0] >= (double)tf[r];  // NaN never passes
-    m1[r] = mem[r][1] && mv[r][1] >= (double)tf[r];
-    const uint32_t nm = (m0[r] ? 1u : 0u) + (m1[r] ? 1u : 0u);
-    if (nm) atomicAdd(&S.nmem[r], nm);
-  }
-  __syncthreads();
-  // ---- records, row by row (a row past its member slots selects exactly) ----
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    uint32_t off = 0u;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) off += w < wave ? S.nw[r][w] : 0u;
-    const uint32_t nplain = S.nw[r][0] + S.nw[r][1] + S.nw[r][2] + S.nw[r][3];
-    const uint32_t nmem = S.nmem[r];
-    const int64_t pq = (int64_t)r * a.parts + part;
-    uint64_t *rrow = a.rec + pq * kListCap;
-    uint4 *mrow4 = a.mrec + pq * kMemSlots;
-    uint32_t np_out = nplain, nm_out = nmem, slow = 0u;
-    auto put_member = [&](uint32_t d, double val, uint32_t id) __attribute__((always_inline)) {
-      uint64_t *w = reinterpret_cast<uint64_t *>(mrow4 + d);
-      w[0] = (uint64_t)__float_as_uint(rd_f32(val)) | ((uint64_t)id << 32);
-      w[1] = (uint64_t)__double_as_longlong(val);
-    };
-    if (nmem <= (uint32_t)kMemSlots) {
-      uint32_t j = off + pre[r];
-      if (k0[r]) rrow[j++] = (uint64_t)__float_as_uint(pv[r][0]) | ((uint64_t)(uint32_t)id0 << 32);
-      if (k1[r]) rrow[j] = (uint64_t)__float_as_uint(pv[r][1]) | ((uint64_t)(uint32_t)(id0 + 1) << 32);
-      if (m0[r]) put_member(atomicAdd(&S.nmw[r], 1u), mv[r][0], (uint32_t)id0);
-      if (m1[r]) put_member(atomicAdd(&S.nmw[r], 1u), mv[r][1], (uint32_t)(id0 + 1));
-    } else {
-      // more members above the bound than a part's member slots hold: the
-      // part's exact top k over (value, id), every value computed again
-      const uint32_t *mrow = a.mask ? a.mask + (int64_t)r * a.mask_stride : nullptr;
-      auto for_elems = [&](auto f) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int id = id0 + j;
-          float x = v_in[r][j];
-          if (p[r].softcap > 0.0f) x = softcap_f32(x, p[r].softcap);
-          bool ok = id < vocab && x == x;
-          if (ok && mrow) ok = ((mrow[id >> 5] >> (id & 31)) & 1u) != 0u;
-          double val = (double)x;
-          if (ok && mem[r][j]) val = mv[r][j];
-          ok = ok && val == val;
-          f(key96(val, (uint32_t)id), ok, val, (uint32_t)id, mem[r][j]);
-        }
-      };
-      uint32_t nval = 0u;
-      for_elems([&](const Key96 &, bool ok, double, uint32_t, bool) { nval += ok ? 1u : 0u; });
-      if (tid == 0) S.sel[3] = 0u;
-      __syncthreads();
-      atomicAdd(&S.sel[3], nval);
-      __syncthreads();
-      const uint32_t need = min(S.sel[3], (uint32_t)kr[r]);
-      __syncthreads();
-      if (tid == 0) {
-        S.nx = 0u;
-        S.nmw[r] = 0u;
-      }
-      __syncthreads();
-      if (need > 0u) {
-        const Key96 kth = block_select96(
-            [&](auto f) { for_elems([&](const Key96 &kx, bool ok, double, uint32_t, bool) { f(kx, ok); }); }, need,
-            S.hist, S.sel);
-        for_elems([&](const Key96 &kx, bool ok, double val, uint32_t id, bool member) {
-          if (ok && key_ge(kx, kth)) {
-            if (member) put_member(atomicAdd(&S.nmw[r], 1u), val, id);
-            else rrow[atomicAdd(&S.nx, 1u)] = (uint64_t)__float_as_uint((float)val) | ((uint64_t)id << 32);
-          }
-        });
-      }
-      __syncthreads();
-      np_out = S.nx;
-      nm_out = S.nmw[r];
-      slow = 1u;
-      __syncthreads();  // S.nx and S.sel are reused by the next row
-    }
-    if (tid == 0)
-      a.pinfo[(int64_t)r * pinfo_stride(a.parts) + part] =
-          (uint64_t)(np_out | (nm_out << 16) | (slow ? kPinfoSlow : 0u)) | ((uint64_t)tkey[r] << 32);
-  }
-}
 
 // ---- GGUF heads: the Q8_1 operand on chip, exact integer block dots ----
 
@@ -338,7 +79,7 @@ __device__ __forceinline__ void lds_dwords(const uint32_t *p, uint32_t (&u)[N]) 
 //     block 8 (u / 4) + 4 h + qt, its half lh): the 16 q (4 words each,
 //     quarter after quarter), then -32 x each quarter's sum of q, then each
 //     quarter's d8.
-// One 32-value block per thread per round (q8.js:27-42): amax,
+// Each 32-value block (q8.js:27-42): amax,
 // d = amax / 127, q = round-half-even(x * (1 / d)), the f16 d and d * sum(q).
 template <int kFmt>
 constexpr int kQOpWords = kFmt == SAS_HEAD_Q6_K ? 24 : 12;
@@ -349,52 +90,51 @@ __host__ __device__ constexpr int q_items(int dim) {
 
 template <int R, int kFmt>
 __device__ __forceinline__ void q81_stage(const LmhArgs &L, uint32_t *U) {
-  const int dim = L.dim, nq = dim / 32, rw = q_items<kFmt>(dim) * kQOpWords<kFmt>;
+  const int dim = L.dim, nq = dim / 4, rw = q_items<kFmt>(dim) * kQOpWords<kFmt>;
+  // eight lanes per 32-value block, four values each (nq is a multiple of
+  // 64: every wave is whole, so the lanes of a block are together)
   for (int t = threadIdx.x; t < R * nq; t += kThreads) {
-    const int r = t / nq, b = t - r * nq;
-    const float *h = L.hidden + (int64_t)r * L.hidden_stride + 32 * b;
-    float v[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) v[i] = h[i];
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
-    const float d = amax / 127.0f;
+    const int r = R == 1 ? 0 : t / nq, i = t - r * nq;
+    const int b = i >> 3, e = i & 7;
+    const f32x4u v = *reinterpret_cast<const f32x4u *>(L.hidden + (int64_t)r * L.hidden_stride + 4 * i);
+    // amax is a maximum of non-negative floats (NaNs left out): their bit
+    // patterns order as the values do
+    uint32_t am = __float_as_uint(fmaxf(fmaxf(fmaxf(0.0f, fabsf(v.x)), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    am = max(am, dppx<kDppQuad1032>(am));
+    am = max(am, dppx<kDppQuad2301>(am));
+    am = max(am, dppx<kDppRowHalfMirror>(am));
+    const float d = __uint_as_float(am) / 127.0f;
     const float inv = d > 0.0f ? 1.0f / d : 0.0f;
-    uint32_t w[8];
-    int sum = 0, half = 0;
+    uint32_t x = 0u, sum = 0u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint32_t x = 0u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float xs = v[4 * j + i] * inv;
-        const float rq = xs != xs ? 0.0f : fminf(fmaxf(rintf(xs), -128.0f), 127.0f);
-        const int qi = (int)rq;
-        sum += qi;
-        x |= ((uint32_t)qi & 0xFFu) << (8 * i);
-      }
-      w[j] = x;
-      if (j == 3) half = sum;
+    for (int c = 0; c < 4; ++c) {
+      const float xs = v[c] * inv;
+      const float rq = xs != xs ? 0.0f : fminf(fmaxf(rintf(xs), -128.0f), 127.0f);
+      const int qi = (int)rq;
+      sum += (uint32_t)qi;
+      x |= ((uint32_t)qi & 0xFFu) << (8 * c);
     }
+    sum += dppx<kDppQuad1032>(sum);
+    sum += dppx<kDppQuad2301>(sum);
+    const int half = (int)sum;  // of the lane's 16 values
+    const int all = (int)(sum + dppx<kDppRowHalfMirror>(sum));
     const float d16 = (float)(_Float16)d;
     uint32_t *ur = U + r * rw;
     if constexpr (kFmt == SAS_HEAD_Q6_K) {
       const int sb = b >> 3, hh = (b >> 2) & 1, qt = b & 3;
-#pragma unroll
-      for (int lh = 0; lh < 2; ++lh) {
-        uint32_t *o = ur + (sb * 4 + hh * 2 + lh) * 24;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[4 * qt + j] = w[4 * lh + j];
-        o[16 + qt] = (uint32_t)(-32 * (lh ? sum - half : half));
+      uint32_t *o = ur + (sb * 4 + hh * 2 + (e >> 2)) * 24;
+      o[4 * qt + (e & 3)] = x;
+      if ((e & 3) == 0) {
+        o[16 + qt] = (uint32_t)(-32 * half);
         o[20 + qt] = __float_as_uint(d16);
       }
     } else {
       uint32_t *o = ur + b * 12;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = w[j];
-      o[8] = __float_as_uint(d16);
-      o[9] = __float_as_uint((float)(_Float16)(d * (float)sum));
+      o[e] = x;
+      if (e == 0) {
+        o[8] = __float_as_uint(d16);
+        o[9] = __float_as_uint((float)(_Float16)(d * (float)all));
+      }
     }
   }
 }
@@ -571,63 +311,73 @@ __device__ __forceinline__ void q_terms(const QRaw<kFmt> &x, const QLane<kFmt> &
 }
 
 template <int R, int kFmt>
-__global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L) {
+__global__ __launch_bounds__(kThreads, 2) void lmh_logits_kernel(const LmhArgs L) {
   // bf16: [R][dim] hidden states; GGUF: their Q8_1 operand
   extern __shared__ __attribute__((aligned(16))) float xs[];
-  __shared__ LmhLds<R> S;
-  __shared__ float s_logit[R][kLmhSpan];  // the part's logits, row by row
   // GGUF: each wave's staged rows (8 rows of one stage)
   __shared__ __attribute__((aligned(16))) uint32_t stg[kFmt == SAS_HEAD_BF16 ? 4 : kWaves * 8 * QStage<kFmt>::pitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int part = blockIdx.x;
-  const int base = part * kLmhSpan;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dim = L.dim;
-  const int vocab = L.s.vocab;
-  // ---- the dot products.  Lanes work in groups of 8 on one id: lane g of
-  // the group takes hidden indices 64 c + 8 g .. + 7 (c = 0, 1, ...), so a
-  // group reads whole 128-byte lines of the weight row and a wave eight of
-  // them per load.  Group grp (32 per block) takes ids base + grp + 32 m,
-  // m = 0 .. 15: at each m the block reads 32 consecutive rows.  (GGUF
-  // heads: lane g takes blocks or units g, g + 8, ... of the row.) ----
+  const int vocab = L.vocab;
+  // ---- the wave's ids: groups of 8 consecutive ones, group gw + nw m at
+  // round m; lanes 8 i .. 8 i + 7 take the group's id i.  Lane g of them
+  // takes hidden indices 64 c + 8 g .. + 7 (c = 0, 1, ...; GGUF heads:
+  // blocks or units g, g + 8, ... of the row).  A wave past the last group
+  // computes the last id again and stores nothing. ----
   const int g = lane & 7;
-  const int grp = (wave << 3) | (lane >> 3);
-  LmhPre pre[R];
+  const int gw = (int)blockIdx.x * kWaves + wave, nw = (int)gridDim.x * kWaves;
+  const int groups = (vocab + 7) >> 3;
+  const int rounds = max((groups - gw + nw - 1) / nw, 1);
+  const int idl = 8 * gw + (lane >> 3);  // this lane's id at round 0
+  const int ids = 8 * nw;                // and the ids between rounds
+  // the eight partial sums of a group's id, in one fixed tree: lane 0 of
+  // the group holds ((p0 + p1) + (p2 + p3)) + ((p4 + p5) + (p6 + p7))
+  auto id_done = [&](float (&a)[R], int id) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float v = a[r];
+      v = v + __uint_as_float(dppx<kDppQuad1032>(__float_as_uint(v)));
+      v = v + __uint_as_float(dppx<kDppQuad2301>(__float_as_uint(v)));
+      v = v + __uint_as_float(dppx<kDppRowHalfMirror>(__float_as_uint(v)));
+      if (g == 0 && id < vocab) L.logits[(int64_t)r * L.logits_stride + id] = v;
+      a[r] = 0.0f;
+    }
+  };
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   if constexpr (kFmt == SAS_HEAD_BF16) {
-    const int C = dim / kLmhStep;              // 128-byte steps per weight row
-    constexpr int kQ = 4;                       // steps per batch of loads
-    const int nb = C / kQ;                      // batches per id (dim is a multiple of 256)
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kQ = 4;               // steps (128 bytes of a row) per batch of loads
+    const int nb = dim / (kLmhStep * kQ);  // batches per id (dim is a multiple of 256)
     const uint16_t *W = static_cast<const uint16_t *>(L.weight);
-    auto wrow = [&](int m) __attribute__((always_inline)) {
-      const int id = min(base + grp + 32 * m, vocab - 1);  // loads stay inside the head
-      return W + (int64_t)id * L.weight_stride + 8 * g;
-    };
+    // batches in the flattened order (round, batch): two in flight ahead of
+    // the one computed (past the last: the last again)
     u32x4 nxt[kQ], nx2[kQ];
-    auto load_into = [&](u32x4 (&dst)[kQ], int m, int cb) __attribute__((always_inline)) {
-      const uint16_t *w = wrow(m) + (int64_t)cb * kQ * kLmhStep;
+    int ml = 0, cl = 0;
+    auto load_next = [&](u32x4 (&dst)[kQ]) __attribute__((always_inline)) {
+      const int id = min(idl + ids * ml, vocab - 1);  // loads stay inside the head
+      const uint16_t *w = W + (int64_t)id * L.weight_stride + 8 * g + cl * (kQ * kLmhStep);
 #pragma unroll
       for (int q = 0; q < kQ; ++q) dst[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w + q * kLmhStep));
+      if (++cl == nb) {
+        if (ml + 1 < rounds) {
+          cl = 0;
+          ++ml;
+        } else {
+          cl = nb - 1;
+        }
+      }
     };
-    // batches in the flattened order (m, cb): two in flight ahead of the one computed
-    const int total = (kLmhSpan / 32) * nb;
-    load_into(nxt, 0, 0);
-    if (total > 1) load_into(nx2, nb > 1 ? 0 : 1, nb > 1 ? 1 : 0);
-    // while the first batches are in flight: the epilogue's inputs (read at
-    // the end, loaded now so that no round trip waits after the dot
-    // products) and the rows' hidden states into LDS
-#pragma unroll
-    for (int r = 0; r < R; ++r) lmh_prefetch_range(L.s, r, base + kLmhIds * tid, pre[r]);
+    load_next(nxt);
+    load_next(nx2);
+    // while the first batches are in flight: the rows' hidden states into LDS
     for (int r = 0; r < R; ++r) {
       const float *h = L.hidden + (int64_t)r * L.hidden_stride;
       for (int i = tid; i < dim; i += kThreads) xs[r * dim + i] = h[i];
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r) lmh_prefetch_ids(pre[r]);
     __syncthreads();  // the hidden states are in LDS
-    for (int m = 0; m < kLmhSpan / 32; ++m) {
-      float acc[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    for (int m = 0; m < rounds; ++m) {
       for (int cb = 0; cb < nb; ++cb) {
         u32x4 cur[kQ];
 #pragma unroll
@@ -635,9 +385,7 @@ __global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L)
           cur[q] = nxt[q];
           nxt[q] = nx2[q];
         }
-        // the batch two ahead in flight
-        const int t2 = m * nb + cb + 2;
-        if (t2 < total) load_into(nx2, t2 / nb, t2 - (t2 / nb) * nb);
+        load_next(nx2);
 #pragma unroll
         for (int q = 0; q < kQ; ++q) {
           const int k = (cb * kQ + q) * kLmhStep + 8 * g;  // hidden indices k .. k + 7
@@ -655,34 +403,23 @@ __global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L)
           }
         }
       }
-      // the group's eight partial sums, in one fixed tree: lane 0 of the
-      // group holds ((p0 + p1) + (p2 + p3)) + ((p4 + p5) + (p6 + p7))
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float v = acc[r];
-        v = v + __shfl_xor(v, 1, 64);
-        v = v + __shfl_xor(v, 2, 64);
-        v = v + __shfl_xor(v, 4, 64);
-        if (g == 0) s_logit[r][grp + 32 * m] = v;
-      }
+      id_done(acc, idl + ids * m);
     }
   } else {
     using St = QStage<kFmt>;
-    constexpr int J = St::loads, D = St::depth, NM = kLmhSpan / 32;
-    static_assert(NM % D == 0, "the ring divides a pass over the wave's batches");
+    constexpr int J = St::loads, D = St::depth;
     const uint8_t *W = static_cast<const uint8_t *>(L.weight);
     // items per id: blocks (Q8_0, Q4_0) or 64-value units (Q6_K); lane g
     // takes g, g + 8, ...: item g of each stage of its row
-    const int items = kFmt == SAS_HEAD_Q6_K ? dim / 64 : dim / 32;
+    const int items = q_items<kFmt>(dim);
     const int rowbytes = kFmt == SAS_HEAD_Q6_K ? 210 * (dim / 256) : (kFmt == SAS_HEAD_Q8_0 ? 34 : 18) * (dim / 32);
     const int per = (items + 7) / 8;  // stages per id
-    // Stage (m, c) of the wave: items 8 c .. 8 c + 7 of ids base + 8 wave +
-    // 32 m + 0 .. 7 (this lane: its group's id), m outer, c inner: a row's
-    // stages follow one another, so the line two stages share comes from
-    // L2 the second time.  The loads are plain (cached) loads for that.
+    // Stage (m, c) of the wave: items 8 c .. 8 c + 7 of round m's ids (this
+    // lane: its group's id), m outer, c inner: a row's stages follow one
+    // another, so the line two stages share comes from L2 the second time.
+    // The loads are plain (cached) loads for that.
     const uint32_t rbi = (uint32_t)((wave * 8 + (lane >> 3)) * St::pitch);  // the lane's row copy in stg
     const QLane<kFmt> ln = q_lane<kFmt>(g, rbi);
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     struct Ring {
       u32x4 v[J];
       uint32_t off;  // the stage's first byte in its first chunk; chunks in use << 8
@@ -691,11 +428,13 @@ __global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L)
     // byte offsets into the head are 32-bit (the host checks that it spans
     // less than 4 GiB); the head is 16-byte aligned
     const uint32_t wstride = (uint32_t)L.weight_stride;
-    auto stage_load = [&](int c2, int m2, Ring &s) __attribute__((always_inline)) {
-      const uint32_t id = (uint32_t)min(base + grp + 32 * m2, vocab - 1);  // loads stay inside the head
-      const uint32_t o = id * wstride + (uint32_t)(St::bytes * c2);        // the stage's first byte
+    int cl = 0, ml = 0;  // the next stage to load
+    // Loads the next stage into a slot (past the last stage: the last one again).
+    auto stage_load = [&](Ring &s) __attribute__((always_inline)) {
+      const uint32_t id = (uint32_t)min(idl + ids * ml, vocab - 1);  // loads stay inside the head
+      const uint32_t o = id * wstride + (uint32_t)(St::bytes * cl);  // the stage's first byte
       const uint32_t off = o & 15u;
-      const uint32_t nch = (off + (uint32_t)min(St::bytes, rowbytes - St::bytes * c2) + 15u) >> 4;
+      const uint32_t nch = (off + (uint32_t)min(St::bytes, rowbytes - St::bytes * cl) + 15u) >> 4;
       const uint32_t o16 = o - off;
       // chunks g, g + 8, ... (past the last: the last again, so that every
       // lane loads and no branch splits the loads in flight)
@@ -703,19 +442,19 @@ __global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L)
       for (int j = 0; j < J; ++j)
         s.v[j] = *reinterpret_cast<const u32x4 *>(W + (o16 + 16u * min((uint32_t)(g + 8 * j), nch - 1u)));
       s.off = off | (nch << 8);
-    };
-    int cl = 0, ml = 0;  // the next stage to load
-    auto advance = [&]() __attribute__((always_inline)) {
       if (++cl == per) {
-        cl = 0;
-        ++ml;
+        if (ml + 1 < rounds) {
+          cl = 0;
+          ++ml;
+        } else {
+          cl = per - 1;
+        }
       }
     };
     // the chunks of the stage in slot rs into the row's copy (the wave's LDS
     // operations run in order, so the reads that follow see them and the
     // previous stage's reads came first), then the slot loads the stage D
-    // ahead (past the last stage: the last stage again); returns the
-    // stage's offset
+    // ahead; returns the stage's offset
     auto stage_take = [&](Ring &rs) __attribute__((always_inline)) {
       const uint32_t off = rs.off & 0xFFu, nch = rs.off >> 8;
       __asm__ volatile("" ::: "memory");
@@ -723,392 +462,74 @@ __global__ __launch_bounds__(kThreads, 2) void lmh_parts_kernel(const LmhArgs L)
       for (int j = 0; j < J; ++j)
         *reinterpret_cast<u32x4 *>(stg + rbi + 4u * min((uint32_t)(g + 8 * j), nch - 1u)) = rs.v[j];
       __asm__ volatile("" ::: "memory");
-      const bool more = ml < NM;
-      stage_load(more ? cl : per - 1, more ? ml : NM - 1, rs);
-      advance();
+      stage_load(rs);
       return off;
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      stage_load(cl, ml, ring[d]);  // D <= NM stages: all exist
-      advance();
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) lmh_prefetch_range(L.s, r, base + kLmhIds * tid, pre[r]);
+    for (int d = 0; d < D; ++d) stage_load(ring[d]);
     uint32_t *U = reinterpret_cast<uint32_t *>(xs);
     const int rw = items * kQOpWords<kFmt>;
     q81_stage<R, kFmt>(L, U);
-#pragma unroll
-    for (int r = 0; r < R; ++r) lmh_prefetch_ids(pre[r]);
     __syncthreads();  // the Q8_1 operand is in LDS
-    // an id's eight partial sums, in one fixed tree: lane 0 of the group
-    // holds ((p0 + p1) + (p2 + p3)) + ((p4 + p5) + (p6 + p7))
-    auto id_done = [&](float (&a)[R], int m2) __attribute__((always_inline)) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float v = a[r];
-        v = v + __shfl_xor(v, 1, 64);
-        v = v + __shfl_xor(v, 2, 64);
-        v = v + __shfl_xor(v, 4, 64);
-        if (g == 0) s_logit[r][grp + 32 * m2] = v;
-      }
-    };
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
     int m = 0, c = 0;  // the stage computed
     // the fields of stage t + 1 are read while stage t is computed (after
     // the last stage: the last stage's copy again, unused)
     QRaw<kFmt> cur;
     q_fetch<kFmt>(stg, ln, stage_take(ring[0]), cur);
-    for (int t0 = 0; t0 < NM * per; t0 += D) {
+    while (m < rounds) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         QRaw<kFmt> nxt;
         q_fetch<kFmt>(stg, ln, stage_take(ring[(d + 1) % D]), nxt);
         const int it = 8 * c + g;
-        if (it < items) q_terms<R, kFmt>(cur, ln, QOp{U + it * kQOpWords<kFmt>, rw}, acc);
+        // past the wave's last stage (the ring's length does not divide the
+        // stages) nothing is added: no lane holds an item
+        if (m < rounds && it < items) q_terms<R, kFmt>(cur, ln, QOp{U + it * kQOpWords<kFmt>, rw}, acc);
         cur = nxt;
-        if (c == per - 1) {
-          id_done(acc, m);
-#pragma unroll
-          for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+        if (++c == per) {
+          if (m < rounds) id_done(acc, idl + ids * m);
           c = 0;
           ++m;
-        } else {
-          ++c;
         }
       }
     }
   }
-  __syncthreads();
-  // ---- the epilogue, all rows together: lane t takes ids base + 2 t, + 1 ----
-  const int id0 = base + kLmhIds * tid;
-  float v[R][2];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    v[r][0] = s_logit[r][kLmhIds * tid];
-    v[r][1] = s_logit[r][kLmhIds * tid + 1];
-    if (L.out_logits) {
-      float *o = L.out_logits + (int64_t)r * vocab;
-      if (id0 < vocab) o[id0] = v[r][0];
-      if (id0 + 1 < vocab) o[id0 + 1] = v[r][1];
-    }
-  }
-  lmh_select_rows<R>(L, S, part, v, id0, pre);
 }
 
-// One block per (row, group of kLmhGroup parts).  The records kept are
-// those at or above the group's k-th largest key (round-down keys for the
-// members: a member whose value reaches a key's value has a key that
-// reaches it), so a merge part holds about k records whatever the spread
-// of the parts' bounds.
-__global__ __launch_bounds__(kThreads) void lmh_group_kernel(const LmhArgs L) {
-  __shared__ uint32_t s_np[kLmhGroup], s_nm[kLmhGroup], s_nw[kWaves], s_nmw, s_slow, s_over, s_n;
-  __shared__ uint32_t s_hist[256], s_sel[4];
-  const SampleArgs &a = L.s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row = blockIdx.x / L.gparts, g = blockIdx.x - row * L.gparts;
-  const int q0 = g * kLmhGroup;
-  const int nq = min(kLmhGroup, a.parts - q0);
-  sas_params p = a.params;
-  if (a.row_params) p = load_row_params(a.row_params + row);
-  const bool greedy = !(p.temperature > 0.0);
-  const int k = greedy ? 1 : min(max(p.top_k, 1), SAS_MAX_TOP_K);
-  // ---- every plain and member slot of the group's parts, loaded before
-  // the counts are known (all slots lie inside the parts' records) ----
-  const int q = tid >> 5, s0 = tid & 31;
-  const uint64_t *src = a.rec + ((int64_t)row * a.parts + q0 + min(q, nq - 1)) * kListCap;
-  const uint4 *msrc = a.mrec + ((int64_t)row * a.parts + q0 + min(q, nq - 1)) * kMemSlots;
-  constexpr int kPer = kLmhSpan / 32;                // plain slots per thread
-  constexpr int kMPer = (kMemSlots + 31) / 32;       // member slots per thread
-  static_assert(kPer * 32 <= kListCap, "plain slots inside a part's records");
-  uint64_t rc[kPer];
-  uint4 mr[kMPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) rc[i] = src[s0 + 32 * i];
-#pragma unroll
-  for (int i = 0; i < kMPer; ++i) {
-    const int j = s0 + 32 * i;
-    mr[i] = j < kMemSlots ? msrc[j] : make_uint4(0u, 0u, 0u, 0u);
-  }
-  // ---- the parts' info words: counts, bounds, slow flags ----
-  uint32_t bound = 0u, slow = 0u;
-#pragma unroll
-  for (int q = 0; q < kLmhGroup; ++q) {
-    if (q < nq) {
-      const uint64_t info = a.pinfo[(int64_t)row * pinfo_stride(a.parts) + q0 + q];
-      bound = max(bound, (uint32_t)(info >> 32));
-      slow |= (uint32_t)info & kPinfoSlow;
-      if (tid == 0) {
-        // within the part's slots whatever the word holds
-        s_np[q] = min((uint32_t)info & 0x7FFFu, (uint32_t)kLmhSpan);
-        s_nm[q] = min(((uint32_t)info >> 16) & 0x7FFFu, (uint32_t)kMemSlots);
-      }
-    }
-  }
-  if (tid == 0) {
-    s_nmw = 0u;
-    s_over = 0u;
-    s_n = 0u;
-    s_slow = slow ? 1u : 0u;
-  }
-  __syncthreads();
-  // the largest part bound: that part alone holds k values above it, and
-  // every part recorded every value at or above its own (smaller) bound
-  const uint32_t bkey = bound > 0x007FFFFFu ? bound : 0u;
-  const int64_t gq = (int64_t)row * L.gparts + g;
-  uint64_t *grec = L.g_rec + gq * kListCap;
-  uint4 *gmem = L.g_mrec + gq * kMemSlots;
-  // ---- the candidates: slots below the parts' counts, at or above bkey ----
-  const uint32_t npq = q < nq ? s_np[q] : 0u;
-  const uint32_t nmq = q < nq ? s_nm[q] : 0u;
-  uint32_t rk[kPer];  // keys (0: not a candidate)
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const uint32_t j = (uint32_t)(s0 + 32 * i);
-    const uint32_t kk = j < npq ? okey(__uint_as_float((uint32_t)rc[i])) : 0u;
-    rk[i] = kk >= bkey ? kk : 0u;
-  }
-  uint32_t mk[kMPer];
-#pragma unroll
-  for (int i = 0; i < kMPer; ++i) {
-    const uint32_t j = (uint32_t)(s0 + 32 * i);
-    const uint32_t kk = j < nmq ? okey(__uint_as_float(mr[i].x)) : 0u;
-    mk[i] = kk >= bkey ? kk : 0u;
-  }
-  // ---- the group's k-th largest key: a radix select, 8 bits a pass from
-  // the top, each pass an LDS histogram of the keys that match the bits
-  // found so far ----
-  {
-    uint32_t n = 0u;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) n += rk[i] != 0u ? 1u : 0u;
-#pragma unroll
-    for (int i = 0; i < kMPer; ++i) n += mk[i] != 0u ? 1u : 0u;
-    n = wave_sum_u32(n);
-    if (lane == 0) atomicAdd(&s_n, n);
-  }
-  __syncthreads();
-  uint32_t t = bkey;
-  if (s_n > (uint32_t)k) {
-    uint32_t res = 0u, need = (uint32_t)k;
-    for (int pass = 0; pass < 4; ++pass) {
-      const int sh = 24 - 8 * pass;
-      const uint32_t hm = sh == 24 ? 0u : ~0u << (sh + 8);  // the bits found so far
-      s_hist[tid] = 0u;
-      __syncthreads();
-      auto add = [&](uint32_t kk) __attribute__((always_inline)) {
-        if (kk != 0u && (kk & hm) == (res & hm)) atomicAdd(&s_hist[(kk >> sh) & 0xFFu], 1u);
-      };
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) add(rk[i]);
-#pragma unroll
-      for (int i = 0; i < kMPer; ++i) add(mk[i]);
-      __syncthreads();
-      if (wave == 0) {
-        // bins 4 lane .. 4 lane + 3; suf = keys in the bins of this lane and above
-        const uint32_t c0 = s_hist[4 * lane], c1 = s_hist[4 * lane + 1], c2 = s_hist[4 * lane + 2],
-                       c3 = s_hist[4 * lane + 3];
-        const uint32_t s4 = c0 + c1 + c2 + c3;
-        uint32_t suf = s4;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const uint32_t y = (uint32_t)__shfl_down((int)suf, d, 64);
-          if (lane + d < 64) suf += y;
-        }
-        const uint32_t above = suf - s4;
-        if (above < need && need <= suf) {
-          uint32_t acc = above, d;
-          if (acc + c3 >= need) {
-            d = 3;
-          } else if ((acc += c3) + c2 >= need) {
-            d = 2;
-          } else if ((acc += c2) + c1 >= need) {
-            d = 1;
-          } else {
-            acc += c1;
-            d = 0;
-          }
-          s_sel[0] = 4u * (uint32_t)lane + d;
-          s_sel[1] = need - acc;
-        }
-      }
-      __syncthreads();
-      res |= s_sel[0] << sh;
-      need = s_sel[1];
-    }
-    t = res;
-  }
-  // ---- the records at or above t ----
-  uint32_t keep = 0u;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i)
-    if (rk[i] != 0u && rk[i] >= t) keep |= 1u << i;
-  const uint32_t mine = (uint32_t)__popc(keep);
-  uint32_t pre = 0u, tot = 0u;
-#pragma unroll
-  for (int bit = 0; bit < 5; ++bit) {
-    const uint64_t bb = __ballot((mine >> bit) & 1u);
-    pre += lanes_below(bb) << bit;
-    tot += (uint32_t)__popcll(bb) << bit;
-  }
-  if (lane == 0) s_nw[wave] = tot;
-  __syncthreads();
-  uint32_t off = 0u;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) off += w < wave ? s_nw[w] : 0u;
-  const uint32_t nplain = s_nw[0] + s_nw[1] + s_nw[2] + s_nw[3];
-  if (nplain > (uint32_t)kListCap) {
-    if (tid == 0) s_over = 1u;
-  } else {
-    uint32_t j = off + pre;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if ((keep >> i) & 1u) grec[j++] = rc[i];
-  }
-#pragma unroll
-  for (int i = 0; i < kMPer; ++i) {
-    if (mk[i] != 0u && mk[i] >= t) {
-      const uint32_t d = atomicAdd(&s_nmw, 1u);
-      if (d < (uint32_t)kMemSlots) gmem[d] = mr[i];
-      else s_over = 1u;
-    }
-  }
-  __syncthreads();
-  uint32_t np_out = nplain, nm_out = s_nmw;
-  if (s_over) {
-    // more records at the key than a merge part holds (ties): the group's
-    // exact top k over (value, id) from the parts' records
-    auto for_recs = [&](auto f) {
-      for (int i = 0; i < kPer; ++i) {
-        const uint32_t j = (uint32_t)(s0 + 32 * i);
-        const bool ok = j < npq;
-        double v = 0.0;
-        uint32_t id = 0u;
-        if (ok) {
-          const uint64_t r = src[j];
-          v = (double)__uint_as_float((uint32_t)r);
-          id = (uint32_t)(r >> 32);
-        }
-        f(key96(v, id), ok, v, id, false, 0u);
-      }
-      for (int i = 0; i < kMPer; ++i) {
-        const uint32_t j = (uint32_t)(s0 + 32 * i);
-        const bool ok = j < nmq;
-        double v = 0.0;
-        uint32_t id = 0u, kb = 0u;
-        if (ok) {
-          const uint4 m = msrc[j];
-          v = __longlong_as_double((long long)(((uint64_t)m.w << 32) | m.z));
-          id = m.y;
-          kb = m.x;
-        }
-        f(key96(v, id), ok, v, id, true, kb);
-      }
-    };
-    uint32_t nval = 0u;
-    for_recs([&](const Key96 &, bool ok, double, uint32_t, bool, uint32_t) { nval += ok ? 1u : 0u; });
-    if (tid == 0) s_sel[3] = 0u;
-    __syncthreads();
-    atomicAdd(&s_sel[3], nval);
-    __syncthreads();
-    const uint32_t need = min(s_sel[3], (uint32_t)k);
-    __syncthreads();
-    if (tid == 0) {
-      s_nw[0] = 0u;
-      s_nmw = 0u;
-      s_slow = 1u;
-    }
-    __syncthreads();
-    if (need > 0u) {
-      const Key96 kth = block_select96(
-          [&](auto f) {
-            for_recs([&](const Key96 &kx, bool ok, double, uint32_t, bool, uint32_t) { f(kx, ok); });
-          },
-          need, s_hist, s_sel);
-      for_recs([&](const Key96 &kx, bool ok, double v, uint32_t id, bool member, uint32_t kb) {
-        if (ok && key_ge(kx, kth)) {
-          if (member) {
-            const uint64_t db = (uint64_t)__double_as_longlong(v);
-            gmem[atomicAdd(&s_nmw, 1u)] = make_uint4(kb, id, (uint32_t)db, (uint32_t)(db >> 32));
-          } else {
-            grec[atomicAdd(&s_nw[0], 1u)] = (uint64_t)__float_as_uint((float)v) | ((uint64_t)id << 32);
-          }
-        }
-      });
-    }
-    __syncthreads();
-    np_out = s_nw[0];
-    nm_out = s_nmw;
-  }
-  if (tid == 0)
-    L.g_pinfo[(int64_t)row * pinfo_stride(L.gparts) + g] =
-        (uint64_t)(np_out | (nm_out << 16) | (s_slow ? kPinfoSlow : 0u)) | ((uint64_t)max(t, bound) << 32);
-}
-
-size_t lmh_scratch_bytes(int rows, int vocab) {
-  const int parts = (vocab + kLmhSpan - 1) / kLmhSpan;
-  const int gparts = (parts + kLmhGroup - 1) / kLmhGroup;
-  return sample_rec_bytes(rows, parts) + sample_rec_bytes(rows, gparts) + 256;
-}
-
-void lmh_layout(LmhArgs *a, void *scratch) {
-  const int rows = a->s.rows;
-  const int parts = (a->s.vocab + kLmhSpan - 1) / kLmhSpan;
-  const int gparts = (parts + kLmhGroup - 1) / kLmhGroup;
-  uint64_t *p = reinterpret_cast<uint64_t *>(scratch);
-  a->s.parts = parts;
-  a->s.span = kLmhSpan;
-  a->s.rec = p;
-  a->s.mrec = reinterpret_cast<uint4 *>(p + (size_t)rows * parts * kListCap);
-  a->s.pinfo = reinterpret_cast<uint64_t *>(a->s.mrec + (size_t)rows * parts * kMemSlots);
-  uint64_t *g = a->s.pinfo + (size_t)rows * pinfo_stride(parts);
-  g = reinterpret_cast<uint64_t *>((reinterpret_cast<uintptr_t>(g) + 255) & ~uintptr_t(255));
-  a->gparts = gparts;
-  a->g_rec = g;
-  a->g_mrec = reinterpret_cast<uint4 *>(g + (size_t)rows * gparts * kListCap);
-  a->g_pinfo = reinterpret_cast<uint64_t *>(a->g_mrec + (size_t)rows * gparts * kMemSlots);
+int lmh_blocks(int vocab, int cus) {
+  // two blocks per CU, each wave at least one group of 8 ids (three and
+  // four per CU measured within 5 % either way: bf16 262,144 x 2,560 214 /
+  // 215 / 220 us, Q6_K 248,320 x 2,560 at three rows 120 / 125 / 124 us)
+  const int all = (vocab + 8 * kWaves - 1) / (8 * kWaves);
+  return all < 2 * cus ? all : 2 * cus;
 }
 
 template <int R, int kFmt>
-static hipError_t launch_parts(const LmhArgs &a, hipStream_t stream) {
+static hipError_t launch_rows(const LmhArgs &a, hipStream_t stream) {
   // bf16: the f32 hidden rows; GGUF: the packed Q8_1 operand of every row
   const size_t lds = kFmt == SAS_HEAD_BF16 ? (size_t)R * a.dim * sizeof(float)
                                            : (size_t)R * q_items<kFmt>(a.dim) * kQOpWords<kFmt> * sizeof(uint32_t);
-  hipLaunchKernelGGL((lmh_parts_kernel<R, kFmt>), dim3((unsigned)a.s.parts), dim3(kThreads), lds, stream, a);
+  hipLaunchKernelGGL((lmh_logits_kernel<R, kFmt>), dim3((unsigned)a.blocks), dim3(kThreads), lds, stream, a);
   return hipGetLastError();
 }
 
 template <int kFmt>
-static hipError_t launch_parts_rows(const LmhArgs &a, hipStream_t stream) {
-  switch (a.s.rows) {
-    case 1: return launch_parts<1, kFmt>(a, stream);
-    case 2: return launch_parts<2, kFmt>(a, stream);
-    case 3: return launch_parts<3, kFmt>(a, stream);
-    default: return launch_parts<4, kFmt>(a, stream);
+static hipError_t launch_format(const LmhArgs &a, hipStream_t stream) {
+  switch (a.rows) {
+    case 1: return launch_rows<1, kFmt>(a, stream);
+    case 2: return launch_rows<2, kFmt>(a, stream);
+    case 3: return launch_rows<3, kFmt>(a, stream);
+    default: return launch_rows<4, kFmt>(a, stream);
   }
 }
 
-hipError_t launch_lm_head_sample(const LmhArgs &a, bool softcap, hipStream_t stream) {
-  (void)softcap;  // the epilogue reads each row's softcap itself
-  hipError_t e;
+hipError_t launch_lm_head(const LmhArgs &a, hipStream_t stream) {
   switch (a.format) {
-    case SAS_HEAD_Q8_0: e = launch_parts_rows<SAS_HEAD_Q8_0>(a, stream); break;
-    case SAS_HEAD_Q4_0: e = launch_parts_rows<SAS_HEAD_Q4_0>(a, stream); break;
-    case SAS_HEAD_Q6_K: e = launch_parts_rows<SAS_HEAD_Q6_K>(a, stream); break;
-    default: e = launch_parts_rows<SAS_HEAD_BF16>(a, stream); break;
+    case SAS_HEAD_Q8_0: return launch_format<SAS_HEAD_Q8_0>(a, stream);
+    case SAS_HEAD_Q4_0: return launch_format<SAS_HEAD_Q4_0>(a, stream);
+    case SAS_HEAD_Q6_K: return launch_format<SAS_HEAD_Q6_K>(a, stream);
+    default: return launch_format<SAS_HEAD_BF16>(a, stream);
   }
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(lmh_group_kernel, dim3((unsigned)(a.s.rows * a.gparts)), dim3(kThreads), 0, stream, a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  SampleArgs m = a.s;
-  m.rec = a.g_rec;
-  m.mrec = a.g_mrec;
-  m.pinfo = a.g_pinfo;
-  m.parts = a.gparts;
-  m.span = kLmhSpan * kLmhGroup;
-  return launch_merge(m, stream);
 }
 
 }  // namespace sas

@@ -1631,6 +1631,31 @@ static void launch_kernel(const SampleArgs &a, hipStream_t stream) {
                        dim3(kThreads), 0, stream, a);
 }
 
+// Record slots per thread for the merge: a part emits about k to 2 k
+// records (its bound certifies k of its own values; ties and the bound's
+// slack add more), so the first 2 k + 8 slots hold nearly every part's
+// records.  Per-row parameters are unknown here: the most slots.
+static int merge_slots(const SampleArgs &a) {
+  if (a.row_params) return kMRMax;
+  const bool greedy = !(a.params.temperature > 0.0);
+  const int k = greedy ? 1 : std::min(std::max(a.params.top_k, 1), SAS_MAX_TOP_K);
+  const int G = kThreads / std::max(a.parts, 1);
+  const int want = (2 * k + 8 + G - 1) / G;
+  return want <= 4 ? 4 : want <= 8 ? 8 : kMRMax;
+}
+
+static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
+  if (a.parts < 1 || a.parts > kMaxParts) return hipErrorInvalidValue;  // the merge's count table
+  switch (merge_slots(a)) {
+    case 4: hipLaunchKernelGGL(sample_merge_kernel<4>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
+    case 8: hipLaunchKernelGGL(sample_merge_kernel<8>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
+    default:
+      hipLaunchKernelGGL(sample_merge_kernel<kMRMax>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a);
+      break;
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_sample(const SampleArgs &a, bool softcap, hipStream_t stream) {
   if (a.hb_offs) {
     const int hrows = a.group > 1 ? a.rows / a.group : a.rows;
@@ -1647,31 +1672,6 @@ hipError_t launch_sample(const SampleArgs &a, bool softcap, hipStream_t stream) 
     default: launch_kernel<true, true, true>(a, stream); break;
   }
   return launch_merge(a, stream);
-}
-
-// Record slots per thread for the merge: a part emits about k to 2 k
-// records (its bound certifies k of its own values; ties and the bound's
-// slack add more), so the first 2 k + 8 slots hold nearly every part's
-// records.  Per-row parameters are unknown here: the most slots.
-int merge_slots(const SampleArgs &a) {
-  if (a.row_params) return kMRMax;
-  const bool greedy = !(a.params.temperature > 0.0);
-  const int k = greedy ? 1 : std::min(std::max(a.params.top_k, 1), SAS_MAX_TOP_K);
-  const int G = kThreads / std::max(a.parts, 1);
-  const int want = (2 * k + 8 + G - 1) / G;
-  return want <= 4 ? 4 : want <= 8 ? 8 : kMRMax;
-}
-
-hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
-  if (a.parts < 1 || a.parts > kMaxParts) return hipErrorInvalidValue;  // the merge's count table
-  switch (merge_slots(a)) {
-    case 4: hipLaunchKernelGGL(sample_merge_kernel<4>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
-    case 8: hipLaunchKernelGGL(sample_merge_kernel<8>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
-    default:
-      hipLaunchKernelGGL(sample_merge_kernel<kMRMax>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a);
-      break;
-  }
-  return hipGetLastError();
 }
 
 }  // namespace sas

@@ -90,8 +90,6 @@ struct SampleArgs {
 // (fewer, larger parts) unless the grid would hold fewer than
 // `min_blocks` blocks; at most kMaxParts parts per row.
 void choose_parts(int rows, int vocab, int min_blocks, int *parts, int *span);
-// The merge launch alone (one block per row) over `a`'s records.
-hipError_t launch_merge(const SampleArgs &a, hipStream_t stream);
 // Launches the sampling kernel on `stream`.  softcap: some row may have a
 // softcap (row_params, or params.softcap > 0).
 hipError_t launch_sample(const SampleArgs &a, bool softcap, hipStream_t stream);
@@ -125,36 +123,25 @@ size_t sample_rec_bytes(int rows, int parts);
 hipError_t launch_pad_rows(const float *src, int64_t stride, int vocab, int rows, float *dst, hipStream_t stream);
 
 // --------------------------------------------------------------- lm head --
-// sas_lm_head_sample: one block per part of kLmhSpan ids computes the
-// part's logits for every row (the hidden states staged in LDS, each lane
-// two ids' whole dot products) and writes the part's records as the parts
-// kernel does; a group launch folds kLmhGroup consecutive parts into one
-// part of the merge kernel's records, which then samples as for sas_sample.
-constexpr int kLmhSpan = 512;   // ids per part: two per thread
-constexpr int kLmhGroup = 8;    // parts per merge part (4,096 ids)
-
+// sas_lm_head_sample: the head's f32 logits of every row of the call, then
+// the sampling launches over them.
 struct LmhArgs {
-  SampleArgs s;          // the sampling descriptor; s.rec/mrec/pinfo: the parts' records, s.parts = parts
   const float *hidden;
   int64_t hidden_stride;
-  const void *weight;    // bf16 bits, or GGUF blocks (format)
-  int64_t weight_stride; // elements (bf16) or bytes (GGUF) between rows
-  int32_t format;        // SAS_HEAD_*
+  const void *weight;     // bf16 bits, or GGUF blocks (format)
+  int64_t weight_stride;  // elements (bf16) or bytes (GGUF) between rows
+  float *logits;          // [rows][logits_stride]: out_logits, or the handle's scratch
+  int64_t logits_stride;
+  int32_t format;         // SAS_HEAD_*
   int32_t dim;
-  float *out_logits;     // [rows][vocab] or null
-  // the merge's records: kLmhGroup parts each (laid out as SampleArgs' records)
-  uint64_t *g_rec;
-  uint4 *g_mrec;
-  uint64_t *g_pinfo;
-  int32_t gparts;
+  int32_t vocab;
+  int32_t rows;           // 1..SAS_LMH_MAX_ROWS
+  int32_t blocks;         // lmh_blocks
 };
 
-// Scratch bytes of both record levels for a batch shape.
-size_t lmh_scratch_bytes(int rows, int vocab);
-// Fills the record pointers of `a` from `scratch` (lmh_scratch_bytes bytes).
-void lmh_layout(LmhArgs *a, void *scratch);
-// The three launches (parts with the head, groups, merge), in stream order.
-hipError_t launch_lm_head_sample(const LmhArgs &a, bool softcap, hipStream_t stream);
+// Blocks of the head launch.
+int lmh_blocks(int vocab, int cus);
+hipError_t launch_lm_head(const LmhArgs &a, hipStream_t stream);
 
 // ---------------------------------------------------------------- verify --
 // Positions are the rows of target_logits: position p = seq * (L + 1) + j,

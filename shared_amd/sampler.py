@@ -343,8 +343,8 @@ class Sampler:
         """sas_lm_head_sample: the LM head (hidden [rows][>= dim] fp32 times
         weight: [vocab][>= dim] bf16 bits as an int16/uint16 tensor, or with
         fmt = HEAD_Q8_0 / HEAD_Q4_0 / HEAD_Q6_K the GGUF blocks as a
-        [vocab][row bytes] uint8 tensor) with the sampling step fused into its
-        epilogue; kw as for sample_into."""
+        [vocab][row bytes] uint8 tensor) with the sampling step behind
+        it; kw as for sample_into."""
         vocab = int(vocab if vocab is not None else weight.shape[0])
         h = self._head(hidden, weight, dim, out_logits, fmt)
         d = rows_descriptor(hidden, out_ids, vocab=vocab, **kw)

@@ -1,5 +1,5 @@
 """GPU parity of sas_lm_head_sample (the LM head with the sampling step fused
-into its epilogue) through the C ABI:
+behind it) through the C ABI:
   - the head's logits (out_logits) bit-exact with the oracle's summation
     order (orc_lm_head_logits: eight fused multiply-add chains, a fixed tree);
   - ids, ranked candidates, {k, cut}, probabilities and flags bit-exact with
@@ -323,3 +323,45 @@ def test_fused_head_decode_steps(sampler, fmt):
         assert sampled[r].tolist() == [int(w["ids"][r]) for w in want], f"sampled row {r}"
         assert np.array_equal(ring[r], ring_of(window[r], ring_len)), f"ring row {r}"
     assert np.array_equal(st.next_tokens.cpu().numpy().view(np.uint32), want[-1]["ids"])
+
+# ids per round of the head launch: two blocks of four waves per CU, 8 ids each
+def _ids_per_round():
+    import torch
+    return 2 * torch.cuda.get_device_properties(0).multi_processor_count * 32
+
+
+@pytest.mark.parametrize("fmt", [W.HEAD_BF16, W.HEAD_Q8_0, W.HEAD_Q4_0, W.HEAD_Q6_K])
+@pytest.mark.parametrize("rounds,extra,dim,rows", [(0, 7, 256, 1), (0, 9, 512, 2), (1, -1, 256, 3), (1, 1, 256, 4),
+                                                   (2, 8, 512, 1), (3, 5, 256, 2), (5, -9, 256, 1)])
+def test_rounds_of_the_head_launch(sampler, fmt, rounds, extra, dim, rows):
+    # vocabularies at the edges of a wave's 8 ids and of the launch's rounds;
+    # GGUF stage counts that the ring of four does not divide
+    vocab = rounds * _ids_per_round() + extra
+    make = W.lmh if fmt == W.HEAD_BF16 else lambda **kw: W.lmhq(fmt, **kw)
+    check(sampler, make(rows=rows, vocab=vocab, dim=dim, seed=vocab + dim + fmt, hist=min(200, vocab)),
+          f"{W.HEAD_NAMES[fmt]} rounds {rounds} {extra:+d}")
+
+
+@pytest.mark.parametrize("fmt", [W.HEAD_Q8_0, W.HEAD_Q4_0, W.HEAD_Q6_K])
+def test_quantized_operand_of_special_hidden_states(sampler, fmt):
+    # zero blocks, one value in a block, halves that round to even, subnormal
+    # and huge blocks, NaN and infinities: the Q8_1 operand is the oracle's
+    b = W.lmhq(fmt, rows=2, vocab=500, dim=512, seed=31 + fmt, hist=0, mask=False)
+    h = b.hidden
+    h[0, 0:32] = 0.0
+    h[0, 32:64] = 0.0
+    h[0, 47] = -2.5
+    h[0, 64:96] = np.linspace(-127.0, 127.0, 32).astype(np.float32) + 0.5
+    h[0, 95] = 127.0
+    h[0, 96:128] *= np.float32(1e-41)
+    h[0, 128:160] *= np.float32(1e4)
+    check(sampler, b, f"{W.HEAD_NAMES[fmt]} special blocks")
+    h[1, 5] = np.nan
+    h[1, 100] = np.inf
+    h[1, 200] = -np.inf
+    print(f"[gpu] {W.HEAD_NAMES[fmt]} NaN and infinities", flush=True)
+    g = run_lmh(sampler, b)
+    lo = O.lm_head_q_logits(fmt, h, b.weight_q)
+    assert np.array_equal(np.isnan(g["logits"]), np.isnan(lo))
+    fine = ~np.isnan(lo)
+    assert np.array_equal(g["logits"][fine].view(np.uint32), lo[fine].view(np.uint32))
