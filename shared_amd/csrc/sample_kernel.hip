@@ -76,17 +76,18 @@ __device__ __forceinline__ bool before(double va, uint32_t ia, double vb, uint32
 // each wave's lane maxima, ranks the records at or above the bound exactly
 // by (value desc, id asc) and runs the reference's sample() tail.
 
-// The merge kernel loads kMR plain record slots per thread before the
-// counts are known (between them a part's first kThreads * kMR / parts
-// slots, as whole 128-byte lines); a part's records past them are loaded
-// where they are used.  launch_merge picks kMR from the expected count per
-// part (about 2 k plus a few).
+// The merge kernel's kT threads load kMR plain record slots each before the
+// counts are known (between them a part's first kT * kMR / parts slots, as
+// whole 128-byte lines); a part's records past them are loaded where they
+// are used.  launch_merge picks both from the expected records.
 constexpr int kMRMax = 16;
 constexpr int kSurvCap = 1024;    // survivors the merge ranks
 constexpr uint32_t kInexact = 0x80000000u;  // composite bit: the exact value lies above the key
 
+constexpr int kMergeWaves = 16;   // the most waves of a merge block
+
 struct MergeLds {
-  uint32_t wred[kWaves][4];          // per-wave partial results
+  uint32_t wred[kMergeWaves][4];          // per-wave partial results
   uint64_t s_c[kSurvCap + 8];        // survivors: rank composites (zero padded to a multiple of 8)
   double s_v[kSurvCap];              // and exact values
   uint32_t s_rank[kSurvCap];
@@ -100,9 +101,9 @@ struct MergeLds {
   double t_r[SAS_MAX_TOP_K + 8];     // running draw residuals
   uint32_t m;
   uint32_t p_np[kMaxParts];          // the parts' plain record counts
-  double g_v[kWaves];                // greedy rows: each wave's best (value, id), has-any | slow bits
-  uint32_t g_id[kWaves];
-  uint32_t g_f[kWaves];
+  double g_v[kMergeWaves];           // greedy rows: each wave's best (value, id), has-any | slow bits
+  uint32_t g_id[kMergeWaves];
+  uint32_t g_f[kMergeWaves];
 };
 
 struct MergeOut {
@@ -155,6 +156,26 @@ __device__ __forceinline__ void chain(const double *src, double *dst, int n, dou
   }
 }
 
+// The sum src[0] + ... + src[n - 1] (zero padded to a multiple of 8) in the
+// same order, by every lane: the operands are one LDS broadcast each.
+__device__ __forceinline__ double chain_sum(const double *src, int n) {
+  double run = 0.0;
+  double x[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) x[u] = src[u];
+  for (int i = 0; i < n; i += 8) {
+    const int in = i + 8 < n ? i + 8 : i;
+    double y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) y[u] = src[in + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) run = run + x[u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = y[u];
+  }
+  return run;
+}
+
 // The first index (lanes 0..63 of `lo`, then 64..127 of `hi`) below n whose
 // condition holds, or n.
 __device__ __forceinline__ int first_true(bool c_lo, bool c_hi, int n) {
@@ -204,11 +225,14 @@ __device__ __forceinline__ double wave_scan_d(double x) {
 //   cum_i = (S_i / S_{k-1})(1 + e), |e| <= 2.9e-14, so with
 //   D_i = t_i - fl(top_p t_{k-1}):  |S_{k-1}(cum_i - top_p) - D_i| <= 3.3e-14 S_{k-1}
 //   |r_i - (fl(U t_{cut-1}) - t_i)| <= 3.2e-14 S_{cut-1}
-// A row is taken from the scan when every D_i up to the cut is clear of 0
-// by 1e-13 t_{k-1} and also of the top-p edge test (|cum_i - top_p| < 1e-6),
-// and every residual up to the draw is clear of 0 and of the draw edge test
-// (|r_i| <= 1e-12 s_{cut-1}) by 1e-13 t_{cut-1}: then the sequential chains
-// give the same cut, draw and flags.  Other rows run the chains.
+// A row is taken from the scan when every D_i up to the cut is clear by
+// 1e-13 t_{k-1} of 0 and of the top-p edge test's 1e-6 t_{k-1}
+// (|cum_i - top_p| < 1e-6), and every residual up to the draw is clear of 0
+// and of the draw edge test (|r_i| <= 1e-12 s_{cut-1}) by 1e-13 t_{cut-1}:
+// then the sequential chains give the same cut, draw and flags.  The last
+// candidate's sign is not needed: reached or not, the cut is all k.  (At
+// top_p = 1 that candidate's D is 0 in every row, whose chains took 37 rows
+// of 50,257 ids at k = 128 from 21.0 to 28.3 us.)  Other rows run the chains.
 __device__ __forceinline__ uint32_t sample_tail(MergeLds &ml, int kk, int row, double T, double top_p,
                                                 double u_row, uint32_t flags, const MergeOut &o) {
   const int lane = threadIdx.x & 63;
@@ -245,7 +269,16 @@ __device__ __forceinline__ uint32_t sample_tail(MergeLds &ml, int kk, int row, d
     const double da = ta - tp, db = tb - tp;
     int c = min(first_true(da >= 0.0, db >= 0.0, kk) + 1, kk);
     const double mc = (1e-6 + 1e-13) * tk;
-    bool fast = __ballot((lane < c && fabs(da) < mc) || (lane + 64 < c && fabs(db) < mc)) == 0ull;
+    bool fast = true, te = false;
+    if (__ballot((lane < c && fabs(da) < mc) || (lane + 64 < c && fabs(db) < mc)) != 0ull) {
+      // some mass near top_p: on which side, and inside the edge band?
+      const double m0 = 1e-13 * tk, me = 1e-6 * tk;
+      auto unclear = [&](int i, double dx) __attribute__((always_inline)) {
+        return i < c && ((i < kk - 1 && fabs(dx) < m0) || fabs(fabs(dx) - me) < m0);
+      };
+      fast = __ballot(unclear(lane, da) || unclear(lane + 64, db)) == 0ull;
+      te = __ballot((lane < c && fabs(da) < me) || (lane + 64 < c && fabs(db) < me)) != 0ull;
+    }
     int pk = 0;
     if (fast) {
       const double sub = c - 1 < 64 ? bcast(ta, c - 1) : bcast(tb, c - 65);
@@ -255,9 +288,16 @@ __device__ __forceinline__ uint32_t sample_tail(MergeLds &ml, int kk, int row, d
       const double md = (1e-12 + 1e-13) * sub;
       fast = __ballot((lane <= pk && fabs(ra) <= md) || (lane + 64 <= pk && fabs(rb) <= md)) == 0ull;
     }
-    if (fast && !o.probs) {
+    if (fast) {
       cut = c;
       out_id = ml.t_id[pk];
+      if (te) flags |= SAS_FLAG_TOPP_EDGE;
+      if (o.probs) {
+        wave_lds_sync();  // the weights in t_p
+        const double sum = chain_sum(ml.t_p, kk);
+        q_a = p_a / sum;
+        q_b = p_b / sum;
+      }
     } else {
       wave_lds_sync();  // the weights in t_p
       // the weight sum and its prefixes (tokenizer.js:164-167)
@@ -266,34 +306,29 @@ __device__ __forceinline__ uint32_t sample_tail(MergeLds &ml, int kk, int row, d
       const double sum = ml.t_pre[kk - 1];
       q_a = p_a / sum;
       q_b = p_b / sum;
-      if (fast) {
-        cut = c;
-        out_id = ml.t_id[pk];
-      } else {
-        ml.t_q[lane] = q_a;
-        ml.t_q[lane + 64] = q_b;
-        if (lane < 8) ml.t_q[128 + lane] = 0.0;
-        wave_lds_sync();
-        // top-p (tokenizer.js:169-174): the first i with q_0 + ... + q_i >= top_p
-        if (lane == 0) chain<false>(ml.t_q, ml.t_cum, kk, 0.0);
-        wave_lds_sync();
-        const double c_a = ml.t_cum[lane], c_b = ml.t_cum[lane + 64];
-        cut = min(first_true(c_a >= top_p, c_b >= top_p, kk) + 1, kk);
-        const bool te = __ballot((lane < cut && fabs(c_a - top_p) < 1e-6) ||
-                                 (lane + 64 < cut && fabs(c_b - top_p) < 1e-6)) != 0ull;
-        // the draw (tokenizer.js:175-177): r = U * (p_0 + ... + p_{cut-1}),
-        // minus p_0, p_1, ... until it reaches 0; else the last of the cut
-        const double sub = ml.t_pre[cut - 1];
-        if (lane == 0) chain<true>(ml.t_p, ml.t_r, cut, u_row * sub);
-        wave_lds_sync();
-        const double r_a = ml.t_r[lane], r_b = ml.t_r[lane + 64];
-        const int pick = min(first_true(r_a <= 0.0, r_b <= 0.0, cut), cut - 1);
-        const double eps = 1e-12 * sub;
-        const bool de = __ballot((lane <= pick && fabs(r_a) <= eps) || (lane + 64 <= pick && fabs(r_b) <= eps)) != 0ull;
-        if (te) flags |= SAS_FLAG_TOPP_EDGE;
-        if (de) flags |= SAS_FLAG_DRAW_EDGE;
-        out_id = ml.t_id[pick];
-      }
+      ml.t_q[lane] = q_a;
+      ml.t_q[lane + 64] = q_b;
+      if (lane < 8) ml.t_q[128 + lane] = 0.0;
+      wave_lds_sync();
+      // top-p (tokenizer.js:169-174): the first i with q_0 + ... + q_i >= top_p
+      if (lane == 0) chain<false>(ml.t_q, ml.t_cum, kk, 0.0);
+      wave_lds_sync();
+      const double c_a = ml.t_cum[lane], c_b = ml.t_cum[lane + 64];
+      cut = min(first_true(c_a >= top_p, c_b >= top_p, kk) + 1, kk);
+      const bool te = __ballot((lane < cut && fabs(c_a - top_p) < 1e-6) ||
+                               (lane + 64 < cut && fabs(c_b - top_p) < 1e-6)) != 0ull;
+      // the draw (tokenizer.js:175-177): r = U * (p_0 + ... + p_{cut-1}),
+      // minus p_0, p_1, ... until it reaches 0; else the last of the cut
+      const double sub = ml.t_pre[cut - 1];
+      if (lane == 0) chain<true>(ml.t_p, ml.t_r, cut, u_row * sub);
+      wave_lds_sync();
+      const double r_a = ml.t_r[lane], r_b = ml.t_r[lane + 64];
+      const int pick = min(first_true(r_a <= 0.0, r_b <= 0.0, cut), cut - 1);
+      const double eps = 1e-12 * sub;
+      const bool de = __ballot((lane <= pick && fabs(r_a) <= eps) || (lane + 64 <= pick && fabs(r_b) <= eps)) != 0ull;
+      if (te) flags |= SAS_FLAG_TOPP_EDGE;
+      if (de) flags |= SAS_FLAG_DRAW_EDGE;
+      out_id = ml.t_id[pick];
     }
   }
   if (lane == 0) {
@@ -364,17 +399,18 @@ __device__ __forceinline__ uint4 load_rec4(const uint4 *p) {
 }
 
 // Merge of row `row`: one block.
-template <int kMR>
+template <int kMR, int kT>
 __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int row, const sas_params &p,
                                           uint32_t *s_hist, uint32_t *s_sel) {
   static_assert(kMR >= 1 && kMR <= kMRMax, "record slots per thread");
+  constexpr int kW = kT / 64;  // waves
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int P = a.parts;
   const bool greedy = !(p.temperature > 0.0);
   const int k = greedy ? 1 : min(max(p.top_k, 1), SAS_MAX_TOP_K);
   // Thread (q, sub) = (tid / G, tid % G), G threads per part, reads part
   // q's counts and bound and member record sub of part q.
-  const int G = kThreads / P;
+  const int G = kT / P;
   const int q = tid / G, sub = tid - q * G;
   const bool qok = q < P;
   const int64_t pq = (int64_t)row * P + (qok ? q : 0);
@@ -387,17 +423,17 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
   const uint4 m4 = load_rec4(mq + min(sub, kMemSlots - 1));
   // Plain records: the first 16 Lc slots of every part as whole 128-byte
   // lines.  Lanes 8 g .. 8 g + 7 of a wave read one line, 16 bytes (two
-  // records) each; load i of reader R = 4 g + wave is chunk z = R +
-  // (kThreads / 8) i, line z / P of part z % P.  Readers alternate over the
+  // records) each; load i of reader R = kW g + wave is chunk z = R +
+  // (kT / 8) i, line z / P of part z % P.  Readers alternate over the
   // waves, so that every wave holds a fair share of every part's lines (the
   // bound below takes the weakest wave).  A chunk past the part's Lc lines
   // reads line 0 again, and it is dropped with the slots past the part's
   // count.  (Lanes reading 16-byte pieces of 64 different lines per load
   // took the step longer: each load then asks the cache for 64 lines.)
-  constexpr int kReaders = kThreads / 8, kChunks = kMR / 2;
+  constexpr int kReaders = kT / 8, kChunks = kMR / 2;
   static_assert(kMR % 2 == 0, "records in pairs");
   static_assert(kReaders * kChunks >= kMaxParts, "at least one line of every part");
-  const int R = (lane >> 3) * kWaves + wave, l8 = tid & 7;
+  const int R = (lane >> 3) * kW + wave, l8 = tid & 7;
   const int Lc = min(kReaders * kChunks / P, kListCap / 16);
   const int zdiv = kReaders / P, zmod = kReaders - zdiv * P;  // chunk z + kReaders: part + zmod, line + zdiv
   const uint4 *rb = reinterpret_cast<const uint4 *>(a.rec);
@@ -428,9 +464,9 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
                        : a.seeds      ? pcg_uniform(a.seeds[row], a.st_state[2 * row + 1], 0u)
                                       : a.uniforms[row];
   // padding: ranks after everything (past more survivors, cleared once their count is known)
-  for (int i = tid; i < kSurvCap / 2 + 8; i += kThreads) ml.s_c[i] = 0ull;
-  ml.s_rank[tid] = 0u;
-  ml.s_rank[tid + kThreads] = 0u;
+  for (int i = tid; i < kSurvCap / 2 + 8; i += kT) ml.s_c[i] = 0ull;
+  // (ranks are added up by several threads per survivor only below kT survivors)
+  for (int i = tid; i < min(kT, kSurvCap); i += kT) ml.s_rank[i] = 0u;
   if (tid == 0) ml.m = 0u;
   // plain and member records of part q (within its slots whatever the word holds)
   const uint32_t np = min((uint32_t)info & 0x7FFFu, (uint32_t)kListCap);
@@ -519,7 +555,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
     double v = 0.0;
     uint32_t id = 0u;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < kW; ++w) {
       const uint32_t f = ml.g_f[w];
       sl = sl || (f & 2u) != 0u;
       if ((f & 1u) && (!h || ranks_before(ml.g_v[w], ml.g_id[w], v, id))) {
@@ -554,7 +590,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
   // ---- the bound: at least jw lanes of every wave hold a key at or above
   // the wave's result, so k keys reach the smallest; and every part's bound
   // certifies k values of its own ----
-  const int jw = (k + kWaves - 1) / kWaves;
+  const int jw = (k + kW - 1) / kW;
   {
     const uint32_t tw = wave_jth_largest_key16(kmax, jw), wb = wave_max_u32(bq);
     const uint32_t ws = __ballot(pslow) ? 1u : 0u;
@@ -568,7 +604,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
   uint32_t lo = 0xFFFFFFFFu, pb = 0u;
   bool slow = false;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
+  for (int w = 0; w < kW; ++w) {
     lo = min(lo, ml.wred[w][0]);
     pb = max(pb, ml.wred[w][1]);
     slow = slow || ml.wred[w][2] != 0u;
@@ -683,8 +719,8 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
   }
   const uint32_t m8 = (m + 7u) & ~7u;
   const uint32_t m64 = (m + 63u) & ~63u;
-  const uint32_t groups = m64 >= (uint32_t)kThreads ? 1u : (uint32_t)kThreads / max(m64, 64u);
-  const uint32_t per = (uint32_t)kThreads / groups;
+  const uint32_t groups = m64 >= (uint32_t)kT ? 1u : (uint32_t)kT / max(m64, 64u);
+  const uint32_t per = (uint32_t)kT / groups;
   const uint32_t share = ((m8 + groups - 1u) / groups + 7u) & ~7u;
   if (!exact) {
     // ---- rank by composites; the first k + 1 ranks are kept ----
@@ -707,7 +743,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
       }
     }
     __syncthreads();
-    for (uint32_t i = (uint32_t)tid; i < m; i += kThreads) {
+    for (uint32_t i = (uint32_t)tid; i < m; i += kT) {
       const uint32_t rank = ml.s_rank[i];
       if (rank <= (uint32_t)k) {
         const uint64_t c = ml.s_c[i];
@@ -729,7 +765,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
     if (__ballot(cl) != 0ull) {
       exact = true;
       flags |= SAS_FLAG_SLOW_SELECT;
-      for (uint32_t i = (uint32_t)tid; i < kSurvCap; i += kThreads) ml.s_rank[i] = 0u;
+      for (uint32_t i = (uint32_t)tid; i < kSurvCap; i += kT) ml.s_rank[i] = 0u;
       __syncthreads();
     }
   }
@@ -749,7 +785,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
       }
     }
     __syncthreads();
-    for (uint32_t i = (uint32_t)tid; i < m; i += kThreads) {
+    for (uint32_t i = (uint32_t)tid; i < m; i += kT) {
       const uint32_t rank = ml.s_rank[i];
       if (rank < (uint32_t)k) {
         ml.t_val[rank] = ml.s_v[i];
@@ -769,8 +805,8 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
 // visible).  Block b takes the row whose parts ran on its XCD (the parts
 // kernel gives each XCD a contiguous run of rows), so the records come from
 // that XCD's L2.
-template <int kMR>
-__global__ __launch_bounds__(kThreads) void sample_merge_kernel(const SampleArgs a) {
+template <int kMR, int kT>
+__global__ __launch_bounds__(kT) void sample_merge_kernel(const SampleArgs a) {
   __shared__ MergeLds ml;
   __shared__ uint32_t s_hist[256];
   __shared__ uint32_t s_sel[4];
@@ -800,7 +836,7 @@ __global__ __launch_bounds__(kThreads) void sample_merge_kernel(const SampleArgs
   }
   sas_params p = a.params;
   if (a.row_params) p = load_row_params(a.row_params + (a.group > 1 ? row / a.group : row));
-  merge_row<kMR>(a, ml, row, p, s_hist, s_sel);
+  merge_row<kMR, kT>(a, ml, row, p, s_hist, s_sel);
 }
 
 // The exact-match cascade (kernels.js:328-339): a = 1, next = pick[0];
@@ -1631,28 +1667,34 @@ static void launch_kernel(const SampleArgs &a, hipStream_t stream) {
                        dim3(kThreads), 0, stream, a);
 }
 
-// Record slots per thread for the merge: a part emits about k to 2 k
-// records (its bound certifies k of its own values; ties and the bound's
-// slack add more), so the first 2 k + 8 slots hold nearly every part's
-// records.  Per-row parameters are unknown here: the most slots.
-static int merge_slots(const SampleArgs &a) {
-  if (a.row_params) return kMRMax;
-  const bool greedy = !(a.params.temperature > 0.0);
-  const int k = greedy ? 1 : std::min(std::max(a.params.top_k, 1), SAS_MAX_TOP_K);
-  const int G = kThreads / std::max(a.parts, 1);
-  const int want = (2 * k + 8 + G - 1) / G;
-  return want <= 4 ? 4 : want <= 8 ? 8 : kMRMax;
+template <int kT>
+static void launch_merge_threads(const SampleArgs &a, int slots, hipStream_t stream) {
+  const dim3 grid((unsigned)a.rows), block(kT);
+  if (slots <= 4) hipLaunchKernelGGL((sample_merge_kernel<4, kT>), grid, block, 0, stream, a);
+  else if (slots <= 8 || kT == 1024) hipLaunchKernelGGL((sample_merge_kernel<8, kT>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((sample_merge_kernel<kMRMax, kT>), grid, block, 0, stream, a);
 }
 
+// Threads and record slots per thread of the merge.  A part emits about k to
+// 2 k records (its bound certifies k of its own values; ties and the bound's
+// slack add more), so slots for 2 k + 8 records of every part hold nearly
+// all of them.  Per-row parameters are unknown here: the largest k.
+//
+// A row's records are one block's work: past 2,048 of them 512 threads read
+// and rank them faster (8 rows of 262,144 ids, k = 64: 14.5 -> 9.1 us; one
+// row, k = 20: 7.4 -> 6.8; 128 rows, k = 50: 8.1 -> 8.0), past 10,240 1,024
+// threads (9 rows, k = 128: 53.8, 18.0 with 512, 15.2); below, the barriers
+// of more waves cost more than they save (64 rows of 151,936 ids, k = 40:
+// 6.6 us with 256 threads, 7.2 with 512, 9.8 with 1,024).
 static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
   if (a.parts < 1 || a.parts > kMaxParts) return hipErrorInvalidValue;  // the merge's count table
-  switch (merge_slots(a)) {
-    case 4: hipLaunchKernelGGL(sample_merge_kernel<4>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
-    case 8: hipLaunchKernelGGL(sample_merge_kernel<8>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a); break;
-    default:
-      hipLaunchKernelGGL(sample_merge_kernel<kMRMax>, dim3((unsigned)a.rows), dim3(kThreads), 0, stream, a);
-      break;
-  }
+  const bool greedy = !a.row_params && !(a.params.temperature > 0.0);
+  const int k = greedy ? 1 : a.row_params ? SAS_MAX_TOP_K : std::min(std::max(a.params.top_k, 1), SAS_MAX_TOP_K);
+  const int per = 2 * k + 8, records = per * a.parts;
+  auto slots = [&](int threads) { return (per + threads / a.parts - 1) / (threads / a.parts); };
+  if (greedy || records <= 2048) launch_merge_threads<256>(a, slots(256), stream);
+  else if (records <= 10240) launch_merge_threads<512>(a, slots(512), stream);
+  else launch_merge_threads<1024>(a, slots(1024), stream);
   return hipGetLastError();
 }
 

@@ -494,3 +494,50 @@ def test_random_sweep(sampler):
             print(f"[gpu] random sweep case {case}", flush=True)
         check(sampler, b, row_params=rp,
               label=f"sweep {case}: rows={rows} vocab={vocab} hist={hlen} mask={mask is not None} rp={rp is not None}")
+
+
+@pytest.mark.parametrize("rows,vocab,top_k", [(1, 65536, 12), (1, 65536, 13), (1, 65536, 76), (1, 65536, 77),
+                                              (2, 65536, 128), (64, 65536, 128), (64, 57344, 128), (3, 1024, 128)])
+@pytest.mark.parametrize("levels", [0, 400, 3])
+def test_merge_block_sizes(sampler, rows, vocab, top_k, levels):
+    # the merge's 256 / 512 / 1,024 threads on both sides of their borders
+    # (records expected per row: parts x (2 k + 8), 64 parts at 65,536 ids in
+    # small batches); `levels` distinct values tie, up to more survivors than
+    # the merge ranks
+    p = Params(temperature=1.0, top_k=top_k, top_p=0.97, repetition_penalty=1.2, presence_penalty=0.5)
+    b = _small_batch(700 + top_k + rows, rows=rows, vocab=vocab, params=p, mask_density=0.6, hist=200)
+    if levels:
+        b.logits[:] = np.round(np.clip(b.logits, -9, 9) * (levels / 18.0)) / np.float32(8.0)
+    print(f"[gpu] merge rows={rows} vocab={vocab} top_k={top_k} levels={levels}", flush=True)
+    check(sampler, b)
+    # the same rows with their own parameters (k unknown to the launch)
+    rng = np.random.default_rng(top_k)
+    check(sampler, b, row_params=[Params(temperature=float(rng.choice([0.0, 1.0])), top_k=int(rng.integers(1, 129)),
+                                         top_p=1.0, presence_penalty=0.5) for _ in range(rows)])
+
+
+@pytest.mark.parametrize("top_p", [1.0, 0.5, 0.25, 0.75, 1.0 - 1e-6, 1.0 - 1e-9, 0.0, -1e-7, 2.0, float("nan")])
+@pytest.mark.parametrize("top_k", [4, 64, 65, 128])
+def test_top_p_edges(sampler, top_p, top_k):
+    # running masses at, near and past top_p: equal weights (exact multiples
+    # of 1/4 ... 1/128), a last weight below 1e-13 and 1e-6 of the sum,
+    # weights that underflow to zero, an infinite and a NaN-making row
+    rng = np.random.default_rng(top_k)
+    x = np.full((8, 3000), -1e4, np.float32)
+    ids = rng.permutation(3000)[:top_k]
+    n = len(ids)
+    x[0, ids] = 2.0
+    x[1, ids] = 2.0
+    x[1, ids[-1]] = -28.0 - np.log(n)       # about 1e-13 of the sum
+    x[2, ids] = 2.0
+    x[2, ids[-1]] = 2.0 - np.log(1e6 * (n - 1))  # about 1e-6 of it
+    x[3, ids] = np.linspace(0.0, -900.0, n)
+    x[4, ids] = rng.standard_normal(n)
+    x[5, ids] = 2.0
+    x[5, ids[0]] = np.inf
+    x[6, ids] = 2.0
+    x[6, ids[n // 2:]] = -29.0 - np.log(n)
+    x[7, ids] = rng.standard_normal(n) * 30.0
+    u = np.array([0.5, 1.0 - 2.0**-53, 0.25, 0.0, 0.7, 0.3, 0.999, 0.1])
+    print(f"[gpu] top-p edges top_p={top_p} top_k={top_k}", flush=True)
+    check(sampler, W.Batch("edges", x, Params(temperature=1.0, top_k=top_k, top_p=top_p), uniforms=u))
