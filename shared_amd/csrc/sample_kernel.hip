@@ -54,15 +54,6 @@ constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 
 
 
-// Lane i's double on every lane (i wave-uniform).
-__device__ __forceinline__ double bcast(double x, int i) {
-  const uint64_t b = (uint64_t)__double_as_longlong(x);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, i);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), i);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-
 // (va, ia) ranks before (vb, ib): value desc, then id asc (tokenizer.js:160
 // stable sort of an id-ascending list; kernels.js:1433, 1439 tie rule).
 __device__ __forceinline__ bool before(double va, uint32_t ia, double vb, uint32_t ib) {
@@ -184,29 +175,6 @@ __device__ __forceinline__ int first_true(bool c_lo, bool c_hi, int n) {
   if (a) return __builtin_ctzll(a);
   if (b) return 64 + __builtin_ctzll(b);
   return n;
-}
-
-// A double moved between lanes by DPP (both halves); lanes without a
-// source read +0.0.
-template <int kCtrl, int kRowMask = 0xF>
-__device__ __forceinline__ double dpp0_d(double x) {
-  const uint64_t b = (uint64_t)__double_as_longlong(x);
-  const uint32_t lo = dpp0<kCtrl, kRowMask>((uint32_t)b), hi = dpp0<kCtrl, kRowMask>((uint32_t)(b >> 32));
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// Inclusive prefix sum of a double over the wave (a tree of depth 6):
-// Hillis-Steele within each row of 16 lanes, then the rows' totals carried
-// forward.  Adding the +0.0 of a lane without a source leaves x unchanged
-// (the weights are >= +0.0).
-__device__ __forceinline__ double wave_scan_d(double x) {
-  x = x + dpp0_d<kDppRowShr1>(x);
-  x = x + dpp0_d<kDppRowShr2>(x);
-  x = x + dpp0_d<kDppRowShr4>(x);
-  x = x + dpp0_d<kDppRowShr8>(x);
-  x = x + dpp0_d<kDppRowBcast15, 0xA>(x);
-  x = x + dpp0_d<kDppRowBcast31, 0xC>(x);
-  return x;
 }
 
 // The reference's sample() tail (tokenizer.js:161-177) in double precision

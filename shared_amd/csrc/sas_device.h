@@ -124,36 +124,6 @@ __device__ __forceinline__ double fd_exp(double x) {
   return res;
 }
 
-// e^x for sums of many weights, where the order of the additions already
-// differs from a sequential loop: within 2 ulp of the exact value, with no
-// division.  x = k ln2 + r (|r| <= ln2 / 2, ln2 split in two parts), e^r by
-// its Taylor series to degree 13 (truncation below 2^-60 relative), scaled
-// by 2^k with ldexp (subnormal results included).  x = -inf gives 0; x past
-// 709.78 overflows to +inf; NaN stays NaN.
-__device__ __forceinline__ double exp_sum(double x) {
-  const double inv_ln2 = 1.44269504088896338700e+00;
-  const double ln2_hi = 6.93147180369123816490e-01, ln2_lo = 1.90821492927058770002e-10;
-  const double xc = fmin(fmax(x, -1100.0), 1100.0);
-  const double k = rint(xc * inv_ln2);
-  const double r = fma(-k, ln2_lo, fma(-k, ln2_hi, xc));
-  double p = 1.0 / 6227020800.0;  // 1/13!
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
-  const double res = __builtin_amdgcn_ldexp(p, (int)k);
-  return x == x ? res : x;
-}
-
 // tanh of an fp32 value, rounded once to fp32 from a double-precision
 // evaluation: an odd Taylor polynomial below 2^-9, (e^2x - 1)/(e^2x + 1)
 // with the fdlibm exp above, 1 from 9.5 on.  Only correctly rounded double
@@ -239,12 +209,6 @@ __device__ __forceinline__ uint32_t wave_jth_largest_key16(uint32_t u, int j) {
   return res;
 }
 
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) x = fmaxf(x, __shfl_xor(x, s, 64));
-  return x;
-}
-
 // Best (value, id) over the wave under ranks_before; lanes without a
 // candidate pass have = false.
 __device__ __forceinline__ void wave_best(bool &have, double &v, uint32_t &id) {
@@ -315,6 +279,73 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
 }
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {
   return wave_reduce(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+
+// Lane i's double on every lane (i wave-uniform).
+__device__ __forceinline__ double bcast(double x, int i) {
+  const uint64_t b = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, i);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), i);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// A double moved between lanes by DPP (both halves); lanes without a
+// source read +0.0.
+template <int kCtrl, int kRowMask = 0xF>
+__device__ __forceinline__ double dpp0_d(double x) {
+  const uint64_t b = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = dpp0<kCtrl, kRowMask>((uint32_t)b), hi = dpp0<kCtrl, kRowMask>((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// Inclusive prefix sum of a double over the wave (a tree of depth 6):
+// Hillis-Steele within each row of 16 lanes, then the rows' totals carried
+// forward.  Adding the +0.0 of a lane without a source leaves x unchanged
+// (x >= +0.0).
+__device__ __forceinline__ double wave_scan_d(double x) {
+  x = x + dpp0_d<kDppRowShr1>(x);
+  x = x + dpp0_d<kDppRowShr2>(x);
+  x = x + dpp0_d<kDppRowShr4>(x);
+  x = x + dpp0_d<kDppRowShr8>(x);
+  x = x + dpp0_d<kDppRowBcast15, 0xA>(x);
+  x = x + dpp0_d<kDppRowBcast31, 0xC>(x);
+  return x;
+}
+
+// x of the lane that kCtrl names (every source inside the row).
+template <int kCtrl>
+__device__ __forceinline__ double dppx_d(double x) {
+  const uint64_t b = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = dppx<kCtrl>((uint32_t)b), hi = dppx<kCtrl>((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// Wave-wide reduction of a double: pairs, quads, eights and rows of 16 by
+// DPP, then the four rows' results.  Every lane (and every wave with the
+// same values) ends with the same bits: op is commutative and the tree is
+// fixed.  LDS permutes take over 100 cycles a step, these about 10.
+template <typename Op>
+__device__ __forceinline__ double wave_reduce_d(double x, Op op) {
+  x = op(x, dppx_d<kDppQuad1032>(x));
+  x = op(x, dppx_d<kDppQuad2301>(x));
+  x = op(x, dppx_d<kDppRowHalfMirror>(x));
+  x = op(x, dppx_d<kDppRowMirror>(x));
+  return op(op(bcast(x, 0), bcast(x, 16)), op(bcast(x, 32), bcast(x, 48)));
+}
+__device__ __forceinline__ float wave_max(float x) {
+  auto mv = [](float a, uint32_t b) { return fmaxf(a, __uint_as_float(b)); };
+  x = mv(x, dppx<kDppQuad1032>(__float_as_uint(x)));
+  x = mv(x, dppx<kDppQuad2301>(__float_as_uint(x)));
+  x = mv(x, dppx<kDppRowHalfMirror>(__float_as_uint(x)));
+  x = mv(x, dppx<kDppRowMirror>(__float_as_uint(x)));
+  auto row = [&](int l) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), l)); };
+  return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
+}
+__device__ __forceinline__ double wave_max_d(double x) {
+  return wave_reduce_d(x, [](double a, double b) { return fmax(a, b); });
+}
+__device__ __forceinline__ double wave_sum_d(double x) {
+  return wave_reduce_d(x, [](double a, double b) { return a + b; });
 }
 
 // The value of the wave's first active lane (wave-uniform values).

@@ -163,7 +163,7 @@ struct VerifyArgs {
   int32_t *out_accepted;     // [seqs]
   // Scratch, each written before it is read within one call:
   double *stats;   // [positions][chunks][4]: target max, target sum, draft max, draft sum
-  double *part;    // [seqs][chunks][2]: residual mass, target mass of the decided position
+  double *part;    // [seqs][chunks][4 waves][2]: residual mass, target mass of the decided position
   double *seqrec;  // [seqs][8]: decided position, its target max / sum, draft max / sum
   float *dtok;     // [positions][2]: target and draft logit of the position's draft token (NaN: masked)
   uint32_t *pk_n;  // [positions][chunks][4 waves]: how the statistics pass packed the wave's allowed values
@@ -172,7 +172,6 @@ struct VerifyArgs {
   int32_t seqs;
   int32_t L;
   int32_t chunks;
-  bool aligned;    // both logits arrays start 16-byte aligned and stride % 4 == 0
 };
 
 size_t verify_scratch_bytes(int seqs, int L, int vocab);

@@ -224,3 +224,23 @@ def test_argument_errors(sampler):
         sampler.verify(t, d, ids, u, temperature=0.0)
     with pytest.raises(SasError, match="draft_len"):
         sampler.verify(t, d, torch.zeros((2, 17), dtype=torch.int32, device="cuda"), u)
+
+
+@pytest.mark.parametrize("vocab", [1, 2, 3, 4, 5, 1023, 1024, 1025, 1027, 4095, 5121, 8190, 300_001])
+@pytest.mark.parametrize("density", [None, 0.9, 0.1])
+def test_runs_of_ids_and_extreme_uniforms(sampler, vocab, density):
+    # vocabularies around a wave's 1,024 ids, a chunk's 4,096 and 64 chunks,
+    # not multiples of 4 (rows at every alignment); draws at the first id, past
+    # the last running sum and between; allowed ids of weight 0 (-inf logits,
+    # weights that underflow at a low temperature) are never drawn
+    inp = _random_inp(vocab + 7, 6, 2, vocab, density, T=0.3)
+    rng = np.random.default_rng(vocab)
+    for s in range(6):
+        inp["uniforms"][s, :, 1] = [0.0, 1.0 - 2.0**-53, 0.5, 2.0**-60, 0.999999, 0.25][s]
+        if s % 2 and vocab > 8:
+            inp["uniforms"][s, :, 0] = 1.0 - 2.0**-53
+            inp["target"][3 * s:3 * s + 3, rng.integers(0, vocab, vocab // 8)] = -np.inf
+            inp["draft"][2 * s:2 * s + 2, rng.integers(0, vocab, vocab // 8)] = -np.inf
+            inp["target"][3 * s:3 * s + 3, vocab // 2:] -= np.float32(400.0)
+    # a uniform at 0 or at the end sits on the first or last running sum
+    check(sampler, inp, f"runs vocab {vocab} density {density}", max_edges=2)
