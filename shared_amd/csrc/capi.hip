@@ -52,6 +52,13 @@ int hip_fail(sas_sampler *s, hipError_t e, const char *what) {
 
 hipStream_t pick_stream(sas_sampler *, void *stream) { return reinterpret_cast<hipStream_t>(stream); }
 
+// Whether work on `stream` is being recorded into a graph.
+bool capturing(void *stream) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &cs) == hipSuccess &&
+         cs != hipStreamCaptureStatusNone;
+}
+
 // Grow a scratch buffer to at least `need` bytes.  The buffer it replaces
 // is retired, not freed: launches queued on any stream, and graphs that
 // recorded them, keep a valid address; sas_destroy frees it.  Capacities
@@ -59,9 +66,7 @@ hipStream_t pick_stream(sas_sampler *, void *stream) { return reinterpret_cast<h
 // stream capture nothing is allocated: the call fails and names the fix.
 int grow(sas_sampler *s, void **buf, size_t *cap, size_t need, void *stream, const char *who) {
   if (need <= *cap) return SAS_OK;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &cs) == hipSuccess &&
-      cs != hipStreamCaptureStatusNone)
+  if (capturing(stream))
     return fail(s, SAS_ERR_INVALID,
                 std::string(who) + ": the handle's scratch is too small for this call and the stream is being "
                                    "captured: size it before the capture (sas_reserve_for, or one eager call "
@@ -118,10 +123,11 @@ bool any_softcap(const sas_rows *r) {
 }
 
 // Kernel arguments for a valid descriptor whose record scratch is `recs`
-// (sas::sample_rec_bytes(rows, parts) bytes) and whose logits have already
-// been padded when vocab < 4.
-void fill_args(const sas_rows *r, const float *logits, int64_t logits_stride, int parts, int span, void *recs,
-               sas::SampleArgs *a) {
+// (sas::sample_rec_bytes(rows, parts) bytes; rows: the descriptor's and a
+// speculative round's draft rows) and whose logits have already been padded
+// when vocab < 4.
+void fill_args(const sas_rows *r, const float *logits, int64_t logits_stride, int rows, int parts, int span,
+               void *recs, sas::SampleArgs *a) {
   a->logits = logits;
   a->logits_stride = logits_stride;
   a->mask = r->mask;
@@ -138,10 +144,11 @@ void fill_args(const sas_rows *r, const float *logits, int64_t logits_stride, in
   a->out_counts = r->out_counts;
   a->out_flags = r->out_flags;
   a->rec = reinterpret_cast<uint64_t *>(recs);
-  a->mrec = reinterpret_cast<uint4 *>(a->rec + (size_t)r->rows * parts * sas::kListCap);
-  a->pinfo = reinterpret_cast<uint64_t *>(a->mrec + (size_t)r->rows * parts * (sas::kListCap / 2));
+  a->mrec = reinterpret_cast<uint4 *>(a->rec + (size_t)rows * parts * sas::kListCap);
+  a->pinfo = reinterpret_cast<uint64_t *>(a->mrec + (size_t)rows * parts * (sas::kListCap / 2));
   a->vocab = r->vocab;
-  a->rows = r->rows;
+  a->rows = rows;
+  a->vrows = r->rows;
   a->parts = parts;
   a->span = span;
 }
@@ -192,6 +199,9 @@ struct SpecDraw {
   uint32_t round;
   int group;
   const sas_spec_state *state;  // chained rounds (sas_spec_step), or null
+  const float *draft_logits;    // the round's draft rows (the verify rows' stride), or null,
+  uint32_t *draft_ids;          // their ids
+  int draft_rows;               // and their number (0: none)
 };
 
 // sas_sample, sas_sample_step (st) and the sampling of sas_spec_exact (sp):
@@ -202,8 +212,9 @@ int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char 
   if (int rc = set_device(s)) return rc;
   // at least two blocks per CU: small batches take shorter parts
   int parts = 0, span = 0;
-  sas::choose_parts(r->rows, r->vocab, 2 * s->cus, &parts, &span);
-  if (int rc = ensure_sample_scratch(s, r->rows, parts, stream, who)) return rc;
+  const int rows = r->rows + (sp ? sp->draft_rows : 0);
+  sas::choose_parts(rows, r->vocab, 2 * s->cus, &parts, &span);
+  if (int rc = ensure_sample_scratch(s, rows, parts, stream, who)) return rc;
   const float *logits = r->logits;
   int64_t stride = r->logits_stride;
   if (r->vocab < 4) {
@@ -217,7 +228,7 @@ int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char 
     stride = 4;
   }
   sas::SampleArgs a{};
-  fill_args(r, logits, stride, parts, span, s->recs, &a);
+  fill_args(r, logits, stride, rows, parts, span, s->recs, &a);
   if (st) {
     a.st_state = st->state;
     a.st_sampled = st->sampled;
@@ -232,6 +243,8 @@ int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char 
     a.spec_seeds = sp->seeds;
     a.spec_round = sp->round;
     a.group = sp->group;
+    a.draft_logits = sp->draft_logits;
+    a.draft_ids = sp->draft_ids;
     if (sp->state) {
       // a chained round: each sequence's ring is its history, its state
       // holds its round and whether it is frozen
@@ -481,7 +494,7 @@ int sas_sample_noalloc(int device, const sas_rows *r, void *stream) {
     stride = 4;
   }
   sas::SampleArgs a{};
-  fill_args(r, logits, stride, parts, span, base, &a);
+  fill_args(r, logits, stride, r->rows, parts, span, base, &a);
   e = sas::launch_sample(a, any_softcap(r), st);
   if (e != hipSuccess) return hip_fail(nullptr, e, "sas_sample_noalloc launch");
   return SAS_OK;
@@ -523,7 +536,18 @@ int spec_on(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *st, co
     return fail(s, SAS_ERR_INVALID, w + ": draft_ids, seeds, out_picks and out_accepted are required");
   hipStream_t stream_h = pick_stream(s, stream);
   const int L = r->draft_len;
-  // the drafts: the argmax of every draft row (argmaxMerge, kernels.js:373-401)
+  // The drafts, the argmax of every draft row (argmaxMerge,
+  // kernels.js:373-401), ride in the verify rows' launches; in launches of
+  // their own where the scratch for both does not fit a capture (the
+  // reserved rows are the verify rows) and for rows of fewer than 4 logits.
+  const int draft_rows = r->draft_logits ? r->seqs * L : 0;
+  bool together = draft_rows > 0 && r->vocab >= 4 && (int64_t)r->seqs * (2 * L + 1) * sas::kMaxParts <= INT32_MAX;
+  if (together) {
+    int parts = 0, span = 0;
+    const int rows = r->seqs * (2 * L + 1);
+    sas::choose_parts(rows, r->vocab, 2 * s->cus, &parts, &span);
+    together = sas::sample_rec_bytes(rows, parts) <= s->recs_cap || !capturing(stream);
+  }
   if (r->draft_logits) {
     sas_rows d{};
     d.logits = r->draft_logits;
@@ -536,7 +560,8 @@ int spec_on(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *st, co
     d.params.top_k = 1;
     d.out_ids = r->draft_ids;
     if (const char *m = check_rows(&d)) return fail(s, SAS_ERR_INVALID, w + ": drafts: " + m);
-    if (int rc = sample_on(s, &d, nullptr, (w + " drafts").c_str(), stream)) return rc;
+    if (!together)
+      if (int rc = sample_on(s, &d, nullptr, (w + " drafts").c_str(), stream)) return rc;
   }
   // every verify row, sampled on its own (kernels.js:255-327)
   sas_rows v{};
@@ -556,7 +581,7 @@ int spec_on(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *st, co
   v.row_hints = r->row_hints;
   v.out_ids = r->out_picks;
   if (const char *m = check_rows(&v, true)) return fail(s, SAS_ERR_INVALID, w + ": " + m);
-  const SpecDraw sp{r->seeds, r->round, L + 1, st};
+  const SpecDraw sp{r->seeds, r->round, L + 1, st, r->draft_logits, r->draft_ids, together ? draft_rows : 0};
   if (int rc = sample_on(s, &v, nullptr, who, stream, &sp)) return rc;
   // the cascade (kernels.js:328-339), and a chained round's commit
   // (kernels.js:340-367)

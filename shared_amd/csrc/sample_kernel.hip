@@ -98,7 +98,7 @@ struct MergeLds {
 };
 
 struct MergeOut {
-  uint32_t *ids;
+  uint32_t *id;  // the row's; the others by row
   double *probs;
   uint32_t *cand_ids;
   int32_t *counts;
@@ -300,7 +300,7 @@ __device__ __forceinline__ uint32_t sample_tail(MergeLds &ml, int kk, int row, d
     }
   }
   if (lane == 0) {
-    o.ids[row] = out_id;
+    *o.id = out_id;
     if (o.counts) {
       o.counts[2 * row] = draw ? kk : 0;
       o.counts[2 * row + 1] = draw ? cut : 0;
@@ -369,7 +369,7 @@ __device__ __forceinline__ uint4 load_rec4(const uint4 *p) {
 // Merge of row `row`: one block.
 template <int kMR, int kT>
 __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int row, const sas_params &p,
-                                          uint32_t *s_hist, uint32_t *s_sel) {
+                                          uint32_t *out_id, uint32_t *s_hist, uint32_t *s_sel) {
   static_assert(kMR >= 1 && kMR <= kMRMax, "record slots per thread");
   constexpr int kW = kT / 64;  // waves
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -535,7 +535,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
     const uint32_t tok = h ? id : SAS_NO_TOKEN;
     // the outputs of sample()'s greedy return: no draw, so no candidates
     if (lane == 0) {
-      a.out_ids[row] = tok;
+      *out_id = tok;
       if (a.out_counts) {
         a.out_counts[2 * row] = 0;
         a.out_counts[2 * row + 1] = 0;
@@ -764,7 +764,7 @@ __device__ __forceinline__ void merge_row(const SampleArgs &a, MergeLds &ml, int
   }
   if (wave != 0) return;
   const int kk = (int)min(m, (uint32_t)k);
-  const MergeOut o{a.out_ids, a.out_probs, a.out_cand_ids, a.out_counts, a.out_flags};
+  const MergeOut o{out_id, a.out_probs, a.out_cand_ids, a.out_counts, a.out_flags};
   const uint32_t tok = sample_tail(ml, kk, row, p.temperature, p.top_p, u_row, flags, o);
   if (a.st_state && lane == 0) step_feedback(a, row, tok, false);
 }
@@ -780,8 +780,9 @@ __global__ __launch_bounds__(kT) void sample_merge_kernel(const SampleArgs a) {
   __shared__ uint32_t s_sel[4];
   int row = blockIdx.x;
   if ((a.rows & 7) == 0 && ((a.rows * a.parts) & 7) == 0) row = (row & 7) * (a.rows >> 3) + (row >> 3);
+  const bool draft = row >= a.vrows;
   const bool stopped = a.st_state && a.st_state[2 * row] != 0u;
-  const bool frozen = a.sp_state && a.sp_state[4 * (a.group > 1 ? row / a.group : row)] != 0u;
+  const bool frozen = a.sp_state && !draft && a.sp_state[4 * (a.group > 1 ? row / a.group : row)] != 0u;
   if (stopped || frozen) {
     // a stopped row emits its first stop id (kernels.js:184-185), a frozen
     // sequence's verify row no pick; neither has candidates
@@ -803,8 +804,9 @@ __global__ __launch_bounds__(kT) void sample_merge_kernel(const SampleArgs a) {
     return;
   }
   sas_params p = a.params;
-  if (a.row_params) p = load_row_params(a.row_params + (a.group > 1 ? row / a.group : row));
-  merge_row<kMR, kT>(a, ml, row, p, s_hist, s_sel);
+  if (draft) p.temperature = 0.0;
+  else if (a.row_params) p = load_row_params(a.row_params + (a.group > 1 ? row / a.group : row));
+  merge_row<kMR, kT>(a, ml, row, p, draft ? a.draft_ids + (row - a.vrows) : a.out_ids + row, s_hist, s_sel);
 }
 
 // The exact-match cascade (kernels.js:328-339): a = 1, next = pick[0];
@@ -937,18 +939,26 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
   const int lo = part * a.span;
   const int nids = min(a.span, vocab - lo);  // > 0
 
-  const int srow = a.group > 1 ? row / a.group : row;  // the row's sequence
+  const bool draft = row >= a.vrows;                               // a round's draft row
+  const int srow = draft ? 0 : a.group > 1 ? row / a.group : row;  // the row's sequence
   // a row that already sampled a stop id (sas_sample_step), or a row of a
   // frozen sequence (sas_spec_step), reads nothing
   if (a.st_state && a.st_state[2 * row] != 0u) return;
-  if (a.sp_state && a.sp_state[4 * srow] != 0u) return;
+  if (a.sp_state && !draft && a.sp_state[4 * srow] != 0u) return;
   sas_params p = a.params;
-  if (a.row_params) p = load_row_params(a.row_params + srow);
+  if (a.row_params && !draft) p = load_row_params(a.row_params + srow);
+  if (draft) {
+    p.temperature = 0.0;
+    p.softcap = 0.0f;
+  }
   const bool greedy = !(p.temperature > 0.0);
   const int k = greedy ? 1 : min(max(p.top_k, 1), SAS_MAX_TOP_K);
   const float softcap = kSoftcap ? p.softcap : 0.0f;
-  const float *lrow = a.logits + (int64_t)row * a.logits_stride;
-  const uint32_t *mrow = kMask ? a.mask + (int64_t)row * a.mask_stride : nullptr;
+  const float *lrow =
+      draft ? a.draft_logits + (int64_t)(row - a.vrows) * a.logits_stride : a.logits + (int64_t)row * a.logits_stride;
+  // (a draft row's mask words are row 0's, made all ones when loaded)
+  const uint32_t *mrow = kMask ? a.mask + (int64_t)(draft ? 0 : row) * a.mask_stride : nullptr;
+  const uint32_t mall = draft ? ~0u : 0u;
 
   // ---- history ids (loaded first: the tables fill while the logits load) ----
   const uint32_t *hid = a.hist_ids;
@@ -975,7 +985,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
       h1 = (int)o1;
     }
   }
-  const bool has_hist = kHist && h1 > h0;
+  const bool has_hist = kHist && !draft && h1 > h0;
   uint32_t hpre[kHistPre];
 #pragma unroll
   for (int j = 0; j < kHistPre; ++j) {
@@ -1000,7 +1010,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
     const int nrem = lo + nids - base;
     // the mask word first: the pass's id words are built from it while the
     // logits still arrive, and the slots are then taken in load order
-    if (kMask) mword = mrow[min((base >> 5) + tid, last_word)];
+    if (kMask) mword = mrow[min((base >> 5) + tid, last_word)] | mall;
 #pragma unroll
     for (int f = 0; f < kSlots; ++f) {
       const int e = base + 1024 * f + 4 * tid;
@@ -1365,7 +1375,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
         float x = 0.0f;
         double val = 0.0;
         if (ok) {
-          const uint32_t mw = kMask ? mrow[id >> 5] : ~0u;
+          const uint32_t mw = kMask ? mrow[id >> 5] | mall : ~0u;
           x = lrow[id];
           cnt = has_hist ? hcount(id) : 0u;
           ok = !kMask || ((mw >> (id & 31u)) & 1u);
@@ -1638,9 +1648,10 @@ static void launch_kernel(const SampleArgs &a, hipStream_t stream) {
 template <int kT>
 static void launch_merge_threads(const SampleArgs &a, int slots, hipStream_t stream) {
   const dim3 grid((unsigned)a.rows), block(kT);
+  constexpr int kMost = kT == 1024 ? 8 : kMRMax;
   if (slots <= 4) hipLaunchKernelGGL((sample_merge_kernel<4, kT>), grid, block, 0, stream, a);
-  else if (slots <= 8 || kT == 1024) hipLaunchKernelGGL((sample_merge_kernel<8, kT>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((sample_merge_kernel<kMRMax, kT>), grid, block, 0, stream, a);
+  else if (slots <= 8) hipLaunchKernelGGL((sample_merge_kernel<8, kT>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((sample_merge_kernel<kMost, kT>), grid, block, 0, stream, a);
 }
 
 // Threads and record slots per thread of the merge.  A part emits about k to
@@ -1668,7 +1679,7 @@ static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
 
 hipError_t launch_sample(const SampleArgs &a, bool softcap, hipStream_t stream) {
   if (a.hb_offs) {
-    const int hrows = a.group > 1 ? a.rows / a.group : a.rows;
+    const int hrows = a.group > 1 ? a.vrows / a.group : a.vrows;
     hipLaunchKernelGGL(hist_bucket_kernel, dim3((unsigned)hrows), dim3(kBucketThreads), 0, stream, a);
   }
   switch ((a.mask ? 4 : 0) | (a.hist_ids || a.ring ? 2 : 0) | (softcap ? 1 : 0)) {

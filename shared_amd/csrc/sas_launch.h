@@ -74,6 +74,12 @@ struct SampleArgs {
   // accepted}.  A frozen sequence's rows read nothing; the others draw with
   // their own round; the ring above is then indexed by sequence.
   const uint32_t *sp_state;
+  // A round's draft rows ride in the same launches: rows vrows .. rows - 1
+  // are greedy rows of draft_logits (the same stride) without a mask,
+  // history or softcap, whose ids go to draft_ids.  vrows == rows: none.
+  const float *draft_logits;
+  uint32_t *draft_ids;
+  int32_t vrows;
   // Long histories bucketed by part before the parts kernel: the ids of
   // history row h (a row, or a group's sequence) that fall in part q are
   // hb_ids[hb_offs[h * (parts + 1) + q] .. hb_offs[h * (parts + 1) + q + 1]).

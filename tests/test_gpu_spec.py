@@ -221,3 +221,62 @@ def test_spec_step_argument_errors(sampler):
     state.ring_len = 0
     with pytest.raises(SasError, match="ring_len"):
         sampler.spec_step_into(t, ids, seeds, picks, acc, state)
+
+
+@pytest.mark.parametrize("seqs,vocab,L", [(1, 1, 1), (2, 3, 2), (3, 4, 2), (5, 5, 1), (7, 8193, 3), (1, 151_936, 16),
+                                          (40, 8192, 4)])
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+def test_draft_rows_ride_with_the_verify_rows(sampler, seqs, vocab, L, softcap):
+    # the draft head's rows take the verify rows' launches but not their mask,
+    # history, softcap or parameters: masks that hide the drafts' best ids,
+    # histories of the best ids, NaN rows and ties among draft logits
+    rng = np.random.default_rng(vocab + L)
+    c = W.spec_case(seqs=seqs, vocab=vocab, drafts=L, hist=min(vocab, 40), mask=True, seed=vocab + seqs + L)
+    best = np.argmax(c["draft"], axis=1).reshape(seqs, L)
+    for s in range(seqs):
+        for j in range(L + 1):
+            for d in best[s]:
+                c["mask"][s * (L + 1) + j, d >> 5] &= ~np.uint32(1 << (int(d) & 31)) if rng.random() < 0.5 else \
+                    np.uint32(0xFFFFFFFF)
+        lo, hi = c["hist_offsets"][s], c["hist_offsets"][s + 1]
+        c["hist_ids"][lo:hi][:L] = best[s][:hi - lo]
+    c["draft"][::3, :] = np.round(c["draft"][::3, :])   # ties: the lowest id
+    c["draft"][1::4, ::2] = np.nan
+    if seqs > 2:
+        c["draft"][-1, :] = np.nan                      # no draft: SAS_NO_TOKEN
+    for p in c["seq_params"]:
+        p.softcap = softcap
+    print(f"[gpu] spec riding drafts seqs={seqs} vocab={vocab} L={L} softcap={softcap}", flush=True)
+    check(run_spec(sampler, c), O.spec_exact(c), f"riding {seqs}x{vocab} L{L}")
+
+
+def test_capture_with_the_verify_rows_reserved():
+    # a handle reserved for a round's verify rows alone: its records may not
+    # hold the draft rows too, so a captured round runs them on their own;
+    # every replay equals the eager round
+    import torch
+    from shared_amd import Sampler
+    c = W.spec_case(seqs=1, vocab=151_936, drafts=2, hist=64, seed=5)
+    want = O.spec_exact(c)
+    with Sampler(0) as s:
+        s.reserve(3, 151_936, hist_ids=64)
+        ids = torch.zeros((1, 2), dtype=torch.int32, device="cuda")
+        picks = torch.empty((1, 3), dtype=torch.int32, device="cuda")
+        acc = torch.empty(1, dtype=torch.int32, device="cuda")
+        args = [dev(c["target"]), ids, dev(c["seeds"], torch.int32), picks, acc]
+        kw = dict(draft_logits=dev(c["draft"]), round=c["round"], hist_ids=dev(c["hist_ids"], torch.int32),
+                  hist_offsets=dev(c["hist_offsets"]), seq_params=dev(pack_params(c["seq_params"]).view(np.uint8)),
+                  row_hints=row_hints(c["seq_params"]), stop_ids=dev(c["stop_ids"], torch.int32))
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            s.spec_exact_into(*args, **kw)
+        for rep in range(3):
+            print(f"[gpu] spec replay {rep}", flush=True)
+            for t in (ids, picks, acc):
+                t.fill_(-7)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(ids.cpu().numpy().view(np.uint32), want["draft_ids"])
+            assert np.array_equal(picks.cpu().numpy().view(np.uint32), want["picks"])
+            assert np.array_equal(acc.cpu().numpy(), want["accepted"])
