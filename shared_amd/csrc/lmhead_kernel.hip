@@ -90,50 +90,66 @@ __host__ __device__ constexpr int q_items(int dim) {
 
 template <int R, int kFmt>
 __device__ __forceinline__ void q81_stage(const LmhArgs &L, uint32_t *U) {
-  const int dim = L.dim, nq = dim / 4, rw = q_items<kFmt>(dim) * kQOpWords<kFmt>;
   // eight lanes per 32-value block, four values each (nq is a multiple of
-  // 64: every wave is whole, so the lanes of a block are together)
-  for (int t = threadIdx.x; t < R * nq; t += kThreads) {
-    const int r = R == 1 ? 0 : t / nq, i = t - r * nq;
-    const int b = i >> 3, e = i & 7;
-    const f32x4u v = *reinterpret_cast<const f32x4u *>(L.hidden + (int64_t)r * L.hidden_stride + 4 * i);
-    // amax is a maximum of non-negative floats (NaNs left out): their bit
-    // patterns order as the values do
-    uint32_t am = __float_as_uint(fmaxf(fmaxf(fmaxf(0.0f, fabsf(v.x)), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    am = max(am, dppx<kDppQuad1032>(am));
-    am = max(am, dppx<kDppQuad2301>(am));
-    am = max(am, dppx<kDppRowHalfMirror>(am));
-    const float d = __uint_as_float(am) / 127.0f;
-    const float inv = d > 0.0f ? 1.0f / d : 0.0f;
-    uint32_t x = 0u, sum = 0u;
+  // 64: every wave is whole, so the lanes of a block are together); a thread's
+  // loads of a batch are in flight together, their chains overlap
+  constexpr int kBatch = 4;
+  const int dim = L.dim, nq = dim / 4, rw = q_items<kFmt>(dim) * kQOpWords<kFmt>;
+  for (int t0 = threadIdx.x; t0 < R * nq; t0 += kBatch * kThreads) {
+    f32x4u v[kBatch];
+    int row[kBatch], quad[kBatch];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float xs = v[c] * inv;
-      const float rq = xs != xs ? 0.0f : fminf(fmaxf(rintf(xs), -128.0f), 127.0f);
-      const int qi = (int)rq;
-      sum += (uint32_t)qi;
-      x |= ((uint32_t)qi & 0xFFu) << (8 * c);
+    for (int n = 0; n < kBatch; ++n) {
+      const int t = min(t0 + n * kThreads, R * nq - 1);
+      row[n] = 0;
+#pragma unroll
+      for (int r = 1; r < R; ++r) row[n] += t >= r * nq ? 1 : 0;
+      quad[n] = t - row[n] * nq;
+      v[n] = *reinterpret_cast<const f32x4u *>(L.hidden + (int64_t)row[n] * L.hidden_stride + 4 * quad[n]);
     }
-    sum += dppx<kDppQuad1032>(sum);
-    sum += dppx<kDppQuad2301>(sum);
-    const int half = (int)sum;  // of the lane's 16 values
-    const int all = (int)(sum + dppx<kDppRowHalfMirror>(sum));
-    const float d16 = (float)(_Float16)d;
-    uint32_t *ur = U + r * rw;
-    if constexpr (kFmt == SAS_HEAD_Q6_K) {
-      const int sb = b >> 3, hh = (b >> 2) & 1, qt = b & 3;
-      uint32_t *o = ur + (sb * 4 + hh * 2 + (e >> 2)) * 24;
-      o[4 * qt + (e & 3)] = x;
-      if ((e & 3) == 0) {
-        o[16 + qt] = (uint32_t)(-32 * half);
-        o[20 + qt] = __float_as_uint(d16);
+#pragma unroll
+    for (int n = 0; n < kBatch; ++n) {
+      if (t0 + n * kThreads >= R * nq) break;  // uniform over the wave
+      const int b = quad[n] >> 3, e = quad[n] & 7;
+      // amax is a maximum of non-negative floats (NaNs left out): their bit
+      // patterns order as the values do
+      uint32_t am = __float_as_uint(
+          fmaxf(fmaxf(fmaxf(0.0f, fabsf(v[n].x)), fabsf(v[n].y)), fmaxf(fabsf(v[n].z), fabsf(v[n].w))));
+      am = max(am, dppx<kDppQuad1032>(am));
+      am = max(am, dppx<kDppQuad2301>(am));
+      am = max(am, dppx<kDppRowHalfMirror>(am));
+      const float d = __uint_as_float(am) / 127.0f;
+      const float inv = d > 0.0f ? 1.0f / d : 0.0f;
+      uint32_t x = 0u, sum = 0u;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float xs = v[n][c] * inv;
+        const float rq = xs != xs ? 0.0f : fminf(fmaxf(rintf(xs), -128.0f), 127.0f);
+        const int qi = (int)rq;
+        sum += (uint32_t)qi;
+        x |= ((uint32_t)qi & 0xFFu) << (8 * c);
       }
-    } else {
-      uint32_t *o = ur + b * 12;
-      o[e] = x;
-      if (e == 0) {
-        o[8] = __float_as_uint(d16);
-        o[9] = __float_as_uint((float)(_Float16)(d * (float)all));
+      sum += dppx<kDppQuad1032>(sum);
+      sum += dppx<kDppQuad2301>(sum);
+      const int half = (int)sum;  // of the lane's 16 values
+      const int all = (int)(sum + dppx<kDppRowHalfMirror>(sum));
+      const float d16 = (float)(_Float16)d;
+      uint32_t *ur = U + row[n] * rw;
+      if constexpr (kFmt == SAS_HEAD_Q6_K) {
+        const int sb = b >> 3, hh = (b >> 2) & 1, qt = b & 3;
+        uint32_t *o = ur + (sb * 4 + hh * 2 + (e >> 2)) * 24;
+        o[4 * qt + (e & 3)] = x;
+        if ((e & 3) == 0) {
+          o[16 + qt] = (uint32_t)(-32 * half);
+          o[20 + qt] = __float_as_uint(d16);
+        }
+      } else {
+        uint32_t *o = ur + b * 12;
+        o[e] = x;
+        if (e == 0) {
+          o[8] = __float_as_uint(d16);
+          o[9] = __float_as_uint((float)(_Float16)(d * (float)all));
+        }
       }
     }
   }
