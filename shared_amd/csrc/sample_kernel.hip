@@ -1110,6 +1110,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
   // caps every value and bounds the capped values instead.
   const bool raw_cap = kSoftcap && !kList && softcap > 0.0f && npass == 1;
   bool capped = !raw_cap;  // the registers and lists hold capped values (or the row has no cap)
+  float tfm = 0.0f;        // what the last pass's list entries reach (raw rows: the margin)
   auto run_pass = [&](int base) __attribute__((always_inline)) {
     // the history members of this thread's word
     const uint32_t hb = has_hist ? L.hbits[tid] : 0u;
@@ -1232,11 +1233,13 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
       } else if (tf > -__builtin_inff()) {
         // values whose cap can equal the bound's: the cap rises by 3 ulp of
         // tanh (near 1) over cap 2^-24 / sech^2(b / cap), plus the rounding
-        // of x / cap; the margin is five times that
-        const float ch = coshf(tf / softcap);
-        tf -= softcap * 0x1p-20f * ch * ch + 1e-5f * (1.0f + fabsf(tf));
+        // of x / cap; the margin is five times that, with e^2|b/cap| >=
+        // cosh^2 (b / cap) for 1 / sech^2
+        const float e2 = __builtin_amdgcn_exp2f(2.8853902f * fabsf(tf / softcap));
+        tf -= softcap * 0x1p-20f * e2 + 1e-5f * (1.0f + fabsf(tf));
       }
     }
+    tfm = tf;
     // whole float4s with a value at or above the bound go to the list (one
     // ballot per float4); their values are cut to the final bound at the end
 #pragma unroll
@@ -1281,9 +1284,22 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
   auto cut = [&](uint32_t e, float4 &q, uint32_t &qid) __attribute__((always_inline)) -> uint32_t {
     const bool qin = (uint32_t)lane + e < n_q && n_q <= (uint32_t)kQuadCap;
     q = qin ? L.q_val[qat + e] : make_float4(qnan(), qnan(), qnan(), qnan());
-    if (kSoftcap && !capped)
-      q = make_float4(softcap_f32(q.x, softcap), softcap_f32(q.y, softcap), softcap_f32(q.z, softcap),
-                      softcap_f32(q.w, softcap));
+    if (kSoftcap && !capped) {
+      // only the values that reach the margin are capped, one per lane at a
+      // time (most lanes hold one); the others drop out
+      uint32_t rem = (q.x >= tfm ? 1u : 0u) | (q.y >= tfm ? 2u : 0u) | (q.z >= tfm ? 4u : 0u) | (q.w >= tfm ? 8u : 0u);
+      float4 o = make_float4(qnan(), qnan(), qnan(), qnan());
+      while (__ballot(rem != 0u)) {
+        const uint32_t b = rem & (0u - rem);
+        const float y = softcap_f32(b == 1u ? q.x : b == 2u ? q.y : b == 4u ? q.z : q.w, softcap);
+        o.x = b == 1u ? y : o.x;
+        o.y = b == 2u ? y : o.y;
+        o.z = b == 4u ? y : o.z;
+        o.w = b == 8u ? y : o.w;
+        rem ^= b;
+      }
+      q = o;
+    }
     qid = L.q_base[qat + e];
     uint32_t pm = (q.x >= tff ? 1u : 0u) | (q.y >= tff ? 2u : 0u) | (q.z >= tff ? 4u : 0u) | (q.w >= tff ? 8u : 0u);
     if (kList && has_hist && lower) {

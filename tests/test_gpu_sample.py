@@ -541,3 +541,20 @@ def test_top_p_edges(sampler, top_p, top_k):
     u = np.array([0.5, 1.0 - 2.0**-53, 0.25, 0.0, 0.7, 0.3, 0.999, 0.1])
     print(f"[gpu] top-p edges top_p={top_p} top_k={top_k}", flush=True)
     check(sampler, W.Batch("edges", x, Params(temperature=1.0, top_k=top_k, top_p=top_p), uniforms=u))
+
+
+@pytest.mark.parametrize("top_k", [1, 5, 64, 100, 128])
+def test_softcap_values_in_clusters(sampler, top_k):
+    # the best ids in runs of 1 to 4 consecutive ones (one float4 of a lane
+    # holds up to four values to cap), some within the cap's plateau of each
+    # other, over one and several parts and with members among them
+    p = Params(temperature=1.0, top_k=top_k, top_p=0.95, softcap=30.0, presence_penalty=0.25)
+    b = _small_batch(900 + top_k, rows=6, vocab=20_003, params=p, mask_density=0.9, hist=300)
+    rng = np.random.default_rng(top_k)
+    for r in range(6):
+        for start in rng.integers(0, 5000, 60) * 4:
+            n = int(rng.integers(1, 5))
+            b.logits[r, start:start + n] = np.float32([9.0, 40.0, 90.0, 140.0, 15.0, 149.0][r]) + \
+                rng.random(n).astype(np.float32) * np.float32(1e-3 if r % 2 else 8.0)
+    print(f"[gpu] softcap clusters top_k={top_k}", flush=True)
+    check(sampler, b)
