@@ -558,3 +558,30 @@ def test_softcap_values_in_clusters(sampler, top_k):
                 rng.random(n).astype(np.float32) * np.float32(1e-3 if r % 2 else 8.0)
     print(f"[gpu] softcap clusters top_k={top_k}", flush=True)
     check(sampler, b)
+
+
+def test_calls_take_torchs_current_stream(sampler):
+    # without a stream argument a call goes to the current stream of the
+    # current device, also inside a stream context
+    import torch
+    from shared_amd.sampler import _stream
+    assert (_stream(None).value or 0) == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert _stream(None).value == side.cuda_stream
+        assert _stream(side).value == side.cuda_stream
+    assert (_stream(None).value or 0) == torch.cuda.current_stream().cuda_stream
+
+
+def test_element_types_are_checked_each_time(sampler):
+    # a type that matched before does not let another one through
+    import torch
+    x = torch.zeros((2, 64), device="cuda")
+    ids = torch.empty(2, dtype=torch.int32, device="cuda")
+    mask = torch.full((2, 2), -1, dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        sampler.sample_into(x, ids, mask=mask, params=Params())
+        with pytest.raises(ValueError, match="mask must hold"):
+            sampler.sample_into(x, ids, mask=mask.to(torch.int64), params=Params())
+        with pytest.raises(ValueError, match="uniforms must hold"):
+            sampler.sample_into(x, ids, uniforms=torch.zeros(2, device="cuda"), params=Params(temperature=1.0))
