@@ -469,8 +469,8 @@ def bench_verify(args) -> int:
 
 
 def bench_lm_head(args) -> int:
-    """LMH1 / LMH3: sas_lm_head_sample steps (three launches: the head with
-    the parts pass, the part groups, the merge).  The 1.34 GB head exceeds
+    """LMH1 / LMH3: sas_lm_head_sample steps (three launches: the head's
+    logits, the parts pass over them, the merge).  The 1.34 GB head exceeds
     the Infinity Cache, so one input set is read from HBM every step."""
     import numpy as np
     import torch
@@ -546,7 +546,7 @@ def bench_lm_head(args) -> int:
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic_from_profiles(args.workload, "lm_head"),
                      "head_format": W.HEAD_NAMES[fmt], "head_bytes": int(b.weight.nbytes),
-                     "kernel": "sas::lmh_parts_kernel + lmh_group_kernel + sample_merge_kernel (one step)",
+                     "kernel": "sas::lmh_logits_kernel + sample_parts_kernel + sample_merge_kernel (one step)",
                      "algorithmic_bytes_per_launch": set_bytes},
         "cpu_baseline": base,
     }
