@@ -1513,7 +1513,14 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
 // Parts per row and ids per part: one pass per part (8192 ids), more
 // passes only when the vocabulary needs more than kMaxParts parts; shorter
 // parts (multiples of 1024 ids) when the grid would hold fewer than
-// min_blocks blocks.
+// min_blocks blocks, at most kSplitParts of them: every part adds about 2 k
+// records to the row's merge, one block's work, and a part of half the ids
+// is hardly faster (its launch and loads' latency stay).  64 -> 32 parts, a
+// call: 4 rows of 262,144 ids at k = 40, 128: 12.5 -> 11.7, 25.9 -> 18.7 us;
+// 8 rows with a softcap, k = 64: 19.9 -> 18.3; one row of 151,936 ids at
+// k = 40: 12.4 -> 11.2, greedy 12.0 -> 11.5; 12 rows of 50,257 ids (13 parts
+// either way): 12.0, 12.0.  24 parts: as 32 (151,936 ids greedy 1 % slower).
+constexpr int kSplitParts = 32;
 void choose_parts(int rows, int vocab, int min_blocks, int *parts, int *span) {
   long long s = kSpanPass;
   if ((long long)vocab > (long long)kMaxParts * kSpanPass) {
@@ -1523,7 +1530,7 @@ void choose_parts(int rows, int vocab, int min_blocks, int *parts, int *span) {
   long long pc = ((long long)vocab + s - 1) / s;
   if (s == kSpanPass && rows > 0 && (long long)rows * pc < min_blocks) {
     long long want = ((long long)min_blocks + rows - 1) / rows;
-    if (want > kMaxParts) want = kMaxParts;
+    if (want > kSplitParts) want = kSplitParts;
     long long s2 = ((long long)vocab + want - 1) / want;
     s2 = (s2 + 1023) / 1024 * 1024;
     if (s2 < 1024) s2 = 1024;
@@ -1676,11 +1683,13 @@ static void launch_merge_threads(const SampleArgs &a, int slots, hipStream_t str
 // all of them.  Per-row parameters are unknown here: the largest k.
 //
 // A row's records are one block's work: past 2,048 of them 512 threads read
-// and rank them faster (8 rows of 262,144 ids, k = 64: 14.5 -> 9.1 us; one
-// row, k = 20: 7.4 -> 6.8; 128 rows, k = 50: 8.1 -> 8.0), past 10,240 1,024
-// threads (9 rows, k = 128: 53.8, 18.0 with 512, 15.2); below, the barriers
-// of more waves cost more than they save (64 rows of 151,936 ids, k = 40:
-// 6.6 us with 256 threads, 7.2 with 512, 9.8 with 1,024).
+// and rank them faster (8 rows of 262,144 ids in 64 parts, k = 64: 14.5 ->
+// 9.1 us; 128 rows, k = 50: 8.1 -> 8.0), past 10,240 (40 parts or more) 1,024
+// threads (9 rows in 52 parts, k = 128: 53.8, 18.0 with 512, 15.2); below,
+// the barriers of more waves cost more than they save (64 rows of 151,936
+// ids, k = 40: 6.6 us with 256 threads, 7.2 with 512, 9.8 with 1,024; a call
+// of 8 rows of 262,144 ids in 32 parts, k = 128: 19.5 us with 512, 20.4 with
+// 1,024).
 static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
   if (a.parts < 1 || a.parts > kMaxParts) return hipErrorInvalidValue;  // the merge's count table
   const bool greedy = !a.row_params && !(a.params.temperature > 0.0);

@@ -497,13 +497,15 @@ def test_random_sweep(sampler):
 
 
 @pytest.mark.parametrize("rows,vocab,top_k", [(1, 65536, 12), (1, 65536, 13), (1, 65536, 76), (1, 65536, 77),
-                                              (2, 65536, 128), (64, 65536, 128), (64, 57344, 128), (3, 1024, 128)])
+                                              (1, 65536, 28), (1, 65536, 29), (2, 65536, 128), (64, 65536, 128),
+                                              (64, 57344, 128), (3, 1024, 128), (1, 319488, 127), (1, 319488, 128),
+                                              (1, 319489, 124), (1, 524288, 76), (2, 524288, 77)])
 @pytest.mark.parametrize("levels", [0, 400, 3])
 def test_merge_block_sizes(sampler, rows, vocab, top_k, levels):
     # the merge's 256 / 512 / 1,024 threads on both sides of their borders
-    # (records expected per row: parts x (2 k + 8), 64 parts at 65,536 ids in
-    # small batches); `levels` distinct values tie, up to more survivors than
-    # the merge ranks
+    # (records expected per row: parts x (2 k + 8), 32 parts at 65,536 ids in
+    # small batches, one per 8,192 ids past 262,144); `levels` distinct values
+    # tie, up to more survivors than the merge ranks
     p = Params(temperature=1.0, top_k=top_k, top_p=0.97, repetition_penalty=1.2, presence_penalty=0.5)
     b = _small_batch(700 + top_k + rows, rows=rows, vocab=vocab, params=p, mask_density=0.6, hist=200)
     if levels:
@@ -514,6 +516,17 @@ def test_merge_block_sizes(sampler, rows, vocab, top_k, levels):
     rng = np.random.default_rng(top_k)
     check(sampler, b, row_params=[Params(temperature=float(rng.choice([0.0, 1.0])), top_k=int(rng.integers(1, 129)),
                                          top_p=1.0, presence_penalty=0.5) for _ in range(rows)])
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17])
+@pytest.mark.parametrize("vocab", [32768, 32769, 65535, 262143, 262144, 262145, 270337])
+def test_split_parts(sampler, rows, vocab):
+    # small batches split a row into at most 32 parts of whole 1,024 ids: the
+    # vocabularies at which a part grows and its last one is short or one id,
+    # and the batches at which the split ends
+    p = Params(temperature=1.0, top_k=50, top_p=0.95, repetition_penalty=1.2, softcap=30.0 if rows == 16 else 0.0)
+    print(f"[gpu] split rows={rows} vocab={vocab}", flush=True)
+    check(sampler, _small_batch(1200 + rows, rows=rows, vocab=vocab, params=p, mask_density=0.5, hist=100))
 
 
 @pytest.mark.parametrize("top_p", [1.0, 0.5, 0.25, 0.75, 1.0 - 1e-6, 1.0 - 1e-9, 0.0, -1e-7, 2.0, float("nan")])
