@@ -239,10 +239,12 @@ int sas_reserve(sas_sampler *s, int32_t rows, int32_t vocab);
  * reserve nothing for that entry point. */
 typedef struct sas_reserve_desc {
   int32_t rows;              /* sampling rows of one call: sas_sample, sas_sample_step,
-                                sas_spec_exact's seqs * (draft_len + 1) verify rows */
+                                the seqs * (draft_len + 1) verify rows of sas_spec_exact and
+                                sas_spec_step (their draft rows are counted in) */
   int32_t vocab;             /* 1..SAS_MAX_VOCAB, the vocabulary of every call below */
   int64_t hist_ids;          /* the most history ids of one call (hist_count, or
-                                rows * ring_len for sas_sample_step): long histories
+                                rows * ring_len for sas_sample_step, seqs * ring_len
+                                for sas_spec_step): long histories
                                 (>= 1,024 ids per row) are bucketed in scratch */
   int32_t lm_head_rows;      /* 0, or the rows of sas_lm_head_sample (<= SAS_LMH_MAX_ROWS;
                                 vocab <= SAS_LMH_MAX_VOCAB) */

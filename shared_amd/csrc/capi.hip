@@ -92,6 +92,25 @@ int ensure_sample_scratch(sas_sampler *s, int rows, int parts, void *stream, con
   return grow(s, &s->recs, &s->recs_cap, sas::sample_rec_bytes(rows, parts), stream, who);
 }
 
+// The most record bytes of one call of at most `rows` rows: a smaller batch
+// may split its rows into more parts, and a speculative round's draft rows
+// (L per L + 1 verify rows) ride with its verify rows.
+size_t most_rec_bytes(const sas_sampler *s, int rows, int vocab) {
+  if (rows <= 0) return 0;
+  const int64_t all = (int64_t)rows + (int64_t)rows * SAS_MAX_DRAFT / (SAS_MAX_DRAFT + 1);
+  const int most = (int)std::min<int64_t>(all, INT32_MAX);
+  size_t bytes = 0;
+  auto shape = [&](int n) {
+    int parts = 0, span = 0;
+    sas::choose_parts(n, vocab, 2 * s->cus, &parts, &span);
+    bytes = std::max(bytes, sas::sample_rec_bytes(n, parts));
+  };
+  // from 2 cus rows on the parts no longer depend on the rows
+  for (int n = 1; n <= std::min(most, 2 * s->cus); ++n) shape(n);
+  shape(most);
+  return bytes;
+}
+
 int set_device(sas_sampler *s) {
   hipError_t e = hipSetDevice(s->device);
   return e == hipSuccess ? SAS_OK : hip_fail(s, e, "hipSetDevice");
@@ -430,14 +449,14 @@ int sas_reserve_for(sas_sampler *s, const sas_reserve_desc *d) {
                 "[1, SAS_MAX_DRAFT] with verify_seqs");
   if (int rc = set_device(s)) return rc;
   const char *who = "sas_reserve_for";
-  // the most parts any batch of <= rows rows may pick (a single row)
-  int parts = 0, span = 0;
-  sas::choose_parts(1, d->vocab, 2 * s->cus, &parts, &span);
-  if (int rc = ensure_sample_scratch(s, d->rows, parts, nullptr, who)) return rc;
+  if (int rc = grow(s, &s->recs, &s->recs_cap, most_rec_bytes(s, d->rows, d->vocab), nullptr, who)) return rc;
   if (d->lm_head_rows > 0)
     if (int rc = ensure_lmh_scratch(s, d->lm_head_rows, d->vocab, nullptr, who)) return rc;
   if (d->vocab < 4 && d->rows > 0)
     if (int rc = grow(s, &s->pad, &s->pad_cap, (size_t)d->rows * 16, nullptr, who)) return rc;
+  // the most parts any batch of <= rows rows may pick (a single row)
+  int parts = 0, span = 0;
+  sas::choose_parts(1, d->vocab, 2 * s->cus, &parts, &span);
   if (d->hist_ids >= sas::kBucketMinIds && d->rows > 0)
     if (int rc = grow(s, &s->hb, &s->hb_cap, hb_bytes(d->hist_ids, d->rows, parts), nullptr, who)) return rc;
   if (d->verify_seqs > 0)
@@ -537,9 +556,10 @@ int spec_on(sas_sampler *s, const sas_spec_rows *r, const sas_spec_state *st, co
   hipStream_t stream_h = pick_stream(s, stream);
   const int L = r->draft_len;
   // The drafts, the argmax of every draft row (argmaxMerge,
-  // kernels.js:373-401), ride in the verify rows' launches; in launches of
-  // their own where the scratch for both does not fit a capture (the
-  // reserved rows are the verify rows) and for rows of fewer than 4 logits.
+  // kernels.js:373-401), ride in the verify rows' launches (a handle
+  // reserved for the verify rows holds both); in launches of their own where
+  // the scratch for both does not fit a capture and for rows of fewer than 4
+  // logits.
   const int draft_rows = r->draft_logits ? r->seqs * L : 0;
   bool together = draft_rows > 0 && r->vocab >= 4 && (int64_t)r->seqs * (2 * L + 1) * sas::kMaxParts <= INT32_MAX;
   if (together) {

@@ -250,16 +250,29 @@ def test_draft_rows_ride_with_the_verify_rows(sampler, seqs, vocab, L, softcap):
     check(run_spec(sampler, c), O.spec_exact(c), f"riding {seqs}x{vocab} L{L}")
 
 
-def test_capture_with_the_verify_rows_reserved():
-    # a handle reserved for a round's verify rows alone: its records may not
-    # hold the draft rows too, so a captured round runs them on their own;
-    # every replay equals the eager round
+def graph_nodes(g) -> int:
+    """Nodes of a captured torch.cuda.CUDAGraph(keep_graph=True)."""
+    import ctypes
+    from shared_amd import _capi
+    hip = _capi.load()  # its HIP runtime's symbols are found behind it
+    n = ctypes.c_size_t(0)
+    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    assert hip.hipGraphGetNodes(g.raw_cuda_graph(), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("rows,nodes", [(3, 3), (2, 5)])
+def test_capture_with_the_verify_rows_reserved(rows, nodes):
+    # a round of three verify rows: a handle reserved for them holds the draft
+    # rows too (three launches); records that hold the verify rows only (a
+    # reserve of two rows) run the drafts on their own when captured (five).
+    # Every replay equals the eager round
     import torch
     from shared_amd import Sampler
     c = W.spec_case(seqs=1, vocab=151_936, drafts=2, hist=64, seed=5)
     want = O.spec_exact(c)
     with Sampler(0) as s:
-        s.reserve(3, 151_936, hist_ids=64)
+        s.reserve(rows, 151_936, hist_ids=64)
         ids = torch.zeros((1, 2), dtype=torch.int32, device="cuda")
         picks = torch.empty((1, 3), dtype=torch.int32, device="cuda")
         acc = torch.empty(1, dtype=torch.int32, device="cuda")
@@ -267,9 +280,11 @@ def test_capture_with_the_verify_rows_reserved():
         kw = dict(draft_logits=dev(c["draft"]), round=c["round"], hist_ids=dev(c["hist_ids"], torch.int32),
                   hist_offsets=dev(c["hist_offsets"]), seq_params=dev(pack_params(c["seq_params"]).view(np.uint8)),
                   row_hints=row_hints(c["seq_params"]), stop_ids=dev(c["stop_ids"], torch.int32))
-        g = torch.cuda.CUDAGraph()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
         with torch.cuda.graph(g):
             s.spec_exact_into(*args, **kw)
+        assert graph_nodes(g) == nodes
+        g.instantiate()
         for rep in range(3):
             print(f"[gpu] spec replay {rep}", flush=True)
             for t in (ids, picks, acc):
@@ -280,3 +295,54 @@ def test_capture_with_the_verify_rows_reserved():
             assert np.array_equal(ids.cpu().numpy().view(np.uint32), want["draft_ids"])
             assert np.array_equal(picks.cpu().numpy().view(np.uint32), want["picks"])
             assert np.array_equal(acc.cpu().numpy(), want["accepted"])
+
+
+@pytest.mark.parametrize("seqs,L,vocab", [(1, 2, 50_257), (4, 2, 50_257), (32, 2, 151_936), (1, 16, 151_936),
+                                          (9, 3, 262_144), (32, 2, 8000)])
+def test_reserved_rounds_allocate_nothing(sampler, seqs, L, vocab):
+    """A handle reserved for a round's seqs * (draft_len + 1) verify rows
+    holds its draft rows: the first eager round leaves the device's free
+    memory as it was, and a round captured with no eager call first holds the
+    three launches (parts, merge, cascade)."""
+    import torch
+    from shared_amd import Sampler
+    print(f"[gpu] reserved spec round seqs={seqs} vocab={vocab} L={L}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(vocab + L)
+    t = torch.randn((seqs * (L + 1), vocab), generator=gen, device="cuda") * 3
+    d = torch.randn((seqs * L, vocab), generator=gen, device="cuda") * 3
+    seeds = torch.arange(seqs, dtype=torch.int32, device="cuda")
+    out = [torch.empty((seqs, L), dtype=torch.int32, device="cuda"),
+           torch.empty((seqs, L + 1), dtype=torch.int32, device="cuda"),
+           torch.empty(seqs, dtype=torch.int32, device="cuda")]
+
+    def call(s):
+        s.spec_exact_into(t, out[0], seeds, out[1], out[2], draft_logits=d, params=Params(top_k=20, top_p=0.95))
+
+    def result():
+        torch.cuda.synchronize()
+        got = [x.cpu().numpy() for x in out]
+        for x in out:
+            x.fill_(-7)
+        torch.cuda.synchronize()
+        return got
+
+    call(sampler)  # loads the kernels too
+    want = result()
+    with Sampler(0) as s:
+        s.reserve(seqs * (L + 1), vocab)
+        free = torch.cuda.mem_get_info()[0]
+        call(s)
+        got = result()
+        assert torch.cuda.mem_get_info()[0] == free
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    with Sampler(0) as s:
+        s.reserve(seqs * (L + 1), vocab)
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            call(s)
+        assert graph_nodes(g) == 3
+        g.instantiate()
+        for rep in range(3):
+            g.replay()
+            got = result()
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), f"replay {rep}"
