@@ -26,7 +26,7 @@ struct sas_sampler {
   size_t vscratch_cap = 0;
   void *pad = nullptr;        // rows of fewer than 4 logits, padded to 4
   size_t pad_cap = 0;
-  void *logits = nullptr;     // the LM head's logits (sas_lm_head_sample without out_logits)
+  void *logits = nullptr;     // the LM head's logits (its calls without out_logits)
   size_t logits_cap = 0;
   void *hb = nullptr;         // long histories bucketed by part
   size_t hb_cap = 0;
@@ -92,13 +92,9 @@ int ensure_sample_scratch(sas_sampler *s, int rows, int parts, void *stream, con
   return grow(s, &s->recs, &s->recs_cap, sas::sample_rec_bytes(rows, parts), stream, who);
 }
 
-// The most record bytes of one call of at most `rows` rows: a smaller batch
-// may split its rows into more parts, and a speculative round's draft rows
-// (L per L + 1 verify rows) ride with its verify rows.
+// The most record bytes of one call of at most `rows` rows (a smaller batch
+// may split its rows into more parts).
 size_t most_rec_bytes(const sas_sampler *s, int rows, int vocab) {
-  if (rows <= 0) return 0;
-  const int64_t all = (int64_t)rows + (int64_t)rows * SAS_MAX_DRAFT / (SAS_MAX_DRAFT + 1);
-  const int most = (int)std::min<int64_t>(all, INT32_MAX);
   size_t bytes = 0;
   auto shape = [&](int n) {
     int parts = 0, span = 0;
@@ -106,8 +102,8 @@ size_t most_rec_bytes(const sas_sampler *s, int rows, int vocab) {
     bytes = std::max(bytes, sas::sample_rec_bytes(n, parts));
   };
   // from 2 cus rows on the parts no longer depend on the rows
-  for (int n = 1; n <= std::min(most, 2 * s->cus); ++n) shape(n);
-  shape(most);
+  for (int n = 1; n <= std::min(rows, 2 * s->cus); ++n) shape(n);
+  if (rows > 0) shape(rows);
   return bytes;
 }
 
@@ -300,14 +296,14 @@ int64_t head_row_bytes(int32_t format, int32_t dim) {
 // Floats between the rows of the head's logits in the handle's scratch.
 int64_t lmh_logits_stride(int32_t vocab) { return ((int64_t)vocab + 3) & ~int64_t(3); }
 
-// The scratch of the LM head's calls of at most `rows` rows at `vocab`: the
-// logits and the sampling step's records (parts hold 1,024 ids or more) and
-// padded rows.
-int ensure_lmh_scratch(sas_sampler *s, int rows, int vocab, void *stream, const char *who) {
-  const int parts = std::min(sas::kMaxParts, (vocab + 1023) / 1024);
-  if (int rc = ensure_sample_scratch(s, rows, parts, stream, who)) return rc;
+// The scratch of the LM head's calls: the sampling step's records (rec_bytes),
+// padded rows, and the logits where the caller takes none.
+int ensure_lmh_scratch(sas_sampler *s, int rows, int vocab, size_t rec_bytes, bool logits, void *stream,
+                       const char *who) {
+  if (int rc = grow(s, &s->recs, &s->recs_cap, rec_bytes, stream, who)) return rc;
   if (vocab < 4)
     if (int rc = grow(s, &s->pad, &s->pad_cap, (size_t)rows * 16, stream, who)) return rc;
+  if (!logits) return SAS_OK;
   return grow(s, &s->logits, &s->logits_cap, (size_t)rows * lmh_logits_stride(vocab) * sizeof(float), stream, who);
 }
 
@@ -355,7 +351,11 @@ int lm_head_on(sas_sampler *s, const sas_lm_head *h, const sas_rows *r, const sa
     return fail(s, SAS_ERR_INVALID, w + ": hidden must be 4-byte aligned");
   if (int rc = set_device(s)) return rc;
   // all scratch before the first launch (a capture that lacks some records nothing)
-  if (int rc = ensure_lmh_scratch(s, r->rows, r->vocab, stream, who)) return rc;
+  int parts = 0, span = 0;
+  sas::choose_parts(r->rows, r->vocab, 2 * s->cus, &parts, &span);
+  if (int rc = ensure_lmh_scratch(s, r->rows, r->vocab, sas::sample_rec_bytes(r->rows, parts), !h->out_logits, stream,
+                                  who))
+    return rc;
   sas::LmhArgs a{};
   a.hidden = h->hidden;
   a.hidden_stride = h->hidden_stride;
@@ -449,9 +449,15 @@ int sas_reserve_for(sas_sampler *s, const sas_reserve_desc *d) {
                 "[1, SAS_MAX_DRAFT] with verify_seqs");
   if (int rc = set_device(s)) return rc;
   const char *who = "sas_reserve_for";
-  if (int rc = grow(s, &s->recs, &s->recs_cap, most_rec_bytes(s, d->rows, d->vocab), nullptr, who)) return rc;
+  // a speculative round's draft rows (L per L + 1 verify rows) ride with its
+  // verify rows
+  const int64_t with_drafts = (int64_t)d->rows + (int64_t)d->rows * SAS_MAX_DRAFT / (SAS_MAX_DRAFT + 1);
+  const size_t recs = most_rec_bytes(s, (int)std::min<int64_t>(with_drafts, INT32_MAX), d->vocab);
+  if (int rc = grow(s, &s->recs, &s->recs_cap, recs, nullptr, who)) return rc;
   if (d->lm_head_rows > 0)
-    if (int rc = ensure_lmh_scratch(s, d->lm_head_rows, d->vocab, nullptr, who)) return rc;
+    if (int rc = ensure_lmh_scratch(s, d->lm_head_rows, d->vocab, most_rec_bytes(s, d->lm_head_rows, d->vocab), true,
+                                    nullptr, who))
+      return rc;
   if (d->vocab < 4 && d->rows > 0)
     if (int rc = grow(s, &s->pad, &s->pad_cap, (size_t)d->rows * 16, nullptr, who)) return rc;
   // the most parts any batch of <= rows rows may pick (a single row)

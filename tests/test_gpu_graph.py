@@ -271,3 +271,39 @@ def test_reserved_handle_captures_with_no_eager_call():
                 err = str(ex)
         torch.cuda.synchronize()
         assert err is not None and "being captured" in err, err
+
+
+def test_head_with_caller_logits_needs_no_logits_scratch():
+    """A handle whose records hold a batch also captures the LM head's calls
+    that bring their own out_logits, with no eager call and no lm_head_rows
+    reserved; without out_logits the call needs the handle's logits."""
+    import torch
+    from shared_amd._capi import SasError
+    b = W.lmh(rows=2, vocab=20_000, dim=512, seed=44, hist=300)
+    print(f"[gpu] graph: lm head with out_logits on a batch's reserve, vocab={b.vocab}", flush=True)
+    hid, wt = to_dev(b.hidden), to_dev(b.weight_bits.view(np.int16))
+    kw = dict(mask=to_dev(b.mask, torch.int32), hist_ids=to_dev(b.hist_ids, torch.int32),
+              hist_offsets=to_dev(b.hist_offsets), uniforms=to_dev(b.uniforms), params=b.params)
+    out = {"ids": torch.empty(b.rows, dtype=torch.int32, device="cuda"),
+           "logits": torch.empty((b.rows, b.vocab), dtype=torch.float32, device="cuda")}
+    with Sampler(0) as e:
+        e.lm_head_sample_into(hid, wt, out["ids"], out_logits=out["logits"], **kw)
+        torch.cuda.synchronize()
+        want = _host(out)
+    with Sampler(0) as s:
+        s.reserve(16, b.vocab)
+        g = _capture(lambda: s.lm_head_sample_into(hid, wt, out["ids"], out_logits=out["logits"], **kw))
+        for rep in range(REPLAYS):
+            _scrub(out)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            _equal(_host(out), want, f"caller logits replay {rep}")
+        err = None
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            try:
+                s.lm_head_sample_into(hid, wt, out["ids"], **kw)
+            except SasError as ex:
+                err = str(ex)
+        torch.cuda.synchronize()
+        assert err is not None and "being captured" in err, err
