@@ -46,7 +46,6 @@ namespace sas {
 
 constexpr int kSlots = kSpanPass / (4 * kThreads);  // float4 per thread per pass
 static_assert(kSlots == 8, "a thread holds 32 values of a pass");
-constexpr int kHashSlots = 512;
 constexpr int kHistPre = 2;                          // history ids per thread loaded before the logits
 constexpr int kQuadCap = 128;                        // float4 entries of one wave's candidate list: two per lane
 static_assert(kQuadCap == 128, "a wave's list is at most two entries per lane at the end");
@@ -889,8 +888,22 @@ static_assert(kXCap >= SAS_MAX_TOP_K, "an exact part selection fits the exact li
 // x_id bit of an exact-selection entry that is a history member
 constexpr uint32_t kXMem = 0x80000000u;
 
+// The hash of a part's history ids: entries of 16 bits each, the id's place
+// in the part and its occurrences, 0 where empty.  Bucketed (long) histories
+// take twice the slots (six blocks per CU still fit).  Where an id finds no
+// slot the members are counted again, in chunks (count_chunk): a few reads of
+// the history, not one per id.  One row of 1,000 ids with 1,000 uniform
+// history ids: 2,460 -> 27 us (512 slots and a scan per missing id before);
+// of 262,144 ids with 8,000 of 8,192 in one part: 2,010 -> 122 us.
+template <bool kList>
+constexpr uint32_t kHashSlots = kList ? 2048 : 1024;
+static_assert(kMaxSpan <= 1 << 16 && SAS_MAX_HISTORY < 1 << 16, "an id's place and occurrences take 16 bits each");
+static_assert(SAS_MAX_VOCAB <= kMaxParts * kMaxSpan, "no part spans more than kMaxSpan ids");
+constexpr int kProbes = 64;  // slots tried for an id
+
+template <bool kList>
 struct PartLds {
-  uint2 hent[kHashSlots];       // (id, count) open-addressing hash of the part's history ids
+  uint32_t hent[kHashSlots<kList>];
   uint32_t hbits[kPassWords];   // history membership of the pass's ids
   uint32_t comb[kPassWords];    // the pass's ids to select from: allowed, not history, inside the part
   uint32_t hmem[kPassWords];    // the pass's allowed history members
@@ -898,11 +911,8 @@ struct PartLds {
   uint32_t q_base[kWaves * kQuadCap];  // and the id of their first value
   double x_val[kXCap];          // exact-valued entries: value, id (| kXMem for a member)
   uint32_t x_id[kXCap];
-  uint32_t hover;               // some history id did not fit in the hash
+  uint32_t hover;               // some history id found no slot in the hash
 };
-
-__device__ __forceinline__ uint32_t hash_slot(uint32_t id) { return (id * 2654435761u) >> 23; }
-static_assert(kHashSlots == 512, "hash_slot yields 9 bits");
 
 // A record store: the merge kernel reads it after the launch boundary, on
 // the same XCD (rows stay on one XCD), so from L2.
@@ -912,7 +922,7 @@ __device__ __forceinline__ void put_rec(uint64_t *p, uint64_t v) { *p = v; }
 // ride in the lists (see `lower`).
 template <bool kMask, bool kHist, bool kSoftcap, bool kList>
 __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6) void sample_parts_kernel(const SampleArgs a) {
-  __shared__ PartLds L;
+  __shared__ __attribute__((aligned(16))) PartLds<kList> L;
   __shared__ uint32_t s_nw[kWaves];   // records of each wave's list
   __shared__ uint32_t s_qover;        // a wave's list overflowed
   __shared__ uint32_t s_thr[kWaves];
@@ -1037,28 +1047,36 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
     const uint32_t off = id - (uint32_t)base;
     if (off < (uint32_t)min(kSpanPass, lo + nids - base)) atomicOr(&L.hbits[off >> 5], 1u << (off & 31u));
   };
+  // an odd factor's low bits: each id of a part of no more ids than slots
+  // has a slot to itself
+  constexpr uint32_t kHS = kHashSlots<kList>;
+  auto slot_of = [&](uint32_t off) __attribute__((always_inline)) { return (off * 2654435761u) & (kHS - 1u); };
+  auto probe_step = [&](uint32_t off) __attribute__((always_inline)) { return ((off * 2654435761u) >> 15) | 1u; };
   if (has_hist) {
-    for (int s = tid; s < kHashSlots; s += kThreads) {
-      L.hent[s] = make_uint2(kEmpty, 0u);
-    }
+    for (uint32_t e = 4u * (uint32_t)tid; e < kHS; e += 4u * (uint32_t)kThreads)
+      *reinterpret_cast<uint4 *>(L.hent + e) = make_uint4(0u, 0u, 0u, 0u);
     L.hbits[tid] = 0u;
     if (tid == 0) L.hover = 0u;
     lds_barrier();
+    int tries = kProbes;  // (none any more once an id of this thread found no slot)
     auto insert = [&](uint32_t id) __attribute__((always_inline)) {
       const uint32_t off = id - (uint32_t)lo;
       if (off >= (uint32_t)nids) return;
       set_bit(id, lo);
-      uint32_t sl = hash_slot(id);
+      uint32_t sl = slot_of(off);
       int probe = 0;
-      for (; probe < kHashSlots; ++probe) {
-        const uint32_t old = atomicCAS(&L.hent[sl].x, kEmpty, id);
-        if (old == kEmpty || old == id) {
-          atomicAdd(&L.hent[sl].y, 1u);
+      for (; probe < tries; ++probe) {
+        const uint32_t old = atomicCAS(&L.hent[sl], 0u, (off << 16) | 1u);
+        if (old == 0u || old >> 16 == off) {  // (one way out: with two, scalars are spilled)
+          atomicAdd(&L.hent[sl], old == 0u ? 0u : 1u);
           break;
         }
-        sl = (sl + 1u) & (uint32_t)(kHashSlots - 1);
+        sl = (sl + probe_step(off)) & (kHS - 1u);
       }
-      if (probe == kHashSlots) L.hover = 1u;
+      if (probe == tries) {
+        tries = 0;
+        L.hover = 1u;
+      }
     };
 #pragma unroll
     for (int j = 0; j < kHistPre; ++j) insert(hpre[j]);
@@ -1075,20 +1093,17 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
     }
     lds_barrier();
   }
-  // occurrences of a history member of the part
-  auto hcount = [&](uint32_t id) __attribute__((always_inline)) -> uint32_t {
-    uint32_t sl = hash_slot(id);
-    for (int probe = 0; probe < kHashSlots; ++probe) {
-      const uint2 e = L.hent[sl];
-      const uint32_t kk = e.x;
-      if (kk == id) return e.y;
-      if (kk == kEmpty) break;
-      sl = (sl + 1u) & (uint32_t)(kHashSlots - 1);
+  // occurrences of the history member at off (wrong where L.hover is set:
+  // the members are then counted again below)
+  auto hcount = [&](uint32_t off) __attribute__((always_inline)) -> uint32_t {
+    uint32_t sl = slot_of(off);
+    for (int probe = 0; probe < kProbes; ++probe) {
+      const uint32_t e = L.hent[sl];
+      if (e == 0u) break;
+      if (e >> 16 == off) return e & 0xFFFFu;
+      sl = (sl + probe_step(off)) & (kHS - 1u);
     }
-    uint32_t c = 0u;
-    if (L.hover)
-      for (int i = h0; i < h1; ++i) c += hid[i] == id ? 1u : 0u;
-    return c;
+    return 0u;
   };
   // ---- passes: values, the bound, the lists ---------------------------------
   // Long (bucketed) histories, whose members are many, with penalties that
@@ -1312,10 +1327,10 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
           const uint32_t id = qid + (uint32_t)c;
           // one pass: the part's history bitmap is still in LDS
           const uint32_t off = id - (uint32_t)lo;
-          const bool member = npass == 1 ? ((L.hbits[off >> 5] >> (off & 31u)) & 1u) != 0u : hcount(id) != 0u;
+          const bool member = npass == 1 ? ((L.hbits[off >> 5] >> (off & 31u)) & 1u) != 0u : hcount(off) != 0u;
           if (member) {
             pm &= ~(1u << c);
-            const double pen = penalize((double)(c == 0 ? q.x : c == 1 ? q.y : c == 2 ? q.z : q.w), hcount(id), p);
+            const double pen = penalize((double)(c == 0 ? q.x : c == 1 ? q.y : c == 2 ? q.z : q.w), hcount(off), p);
             if (pen >= (double)tff) {
               atomicAdd(&s_nxk, 1u);
               const uint32_t d = atomicAdd(&s_nmw, 1u);
@@ -1366,7 +1381,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
     xid = L.x_id[tid];
     // members recorded raw are capped first
     const double xr = L.x_val[tid];
-    xv = penalize(kSoftcap && raw_cap ? (double)softcap_f32((float)xr, softcap) : xr, hcount(xid), p);
+    xv = penalize(kSoftcap && raw_cap ? (double)softcap_f32((float)xr, softcap) : xr, hcount(xid - (uint32_t)lo), p);
     xw = xv >= (double)tff;
     if (xw) atomicAdd(&s_nxk, 1u);
   }
@@ -1376,31 +1391,112 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
   for (int w = 0; w < kWaves; ++w) nw[w] = s_nw[w];
   uint32_t nx = s_nxk;
   uint32_t nxm = nx;  // exact entries that are members (all of them unless the slow selection ran)
+  const bool hover = has_hist && L.hover != 0u;
   const bool overflow = s_qover != 0u || s_nx > (uint32_t)kXCap || nw[0] + nw[1] + nw[2] + nw[3] + nx > (uint32_t)kListCap;
-  if (overflow) {
+  // Some history id found no slot in the hash: the members are gone over
+  // again, and only those that reach the bound are listed.
+  bool exact = overflow;
+  // Without the hash its memory holds 16-bit counters of 2 kHS ids from hc0
+  // on, counted again from the history for each such chunk of the part (a
+  // read of the history per chunk, whatever ids it holds).
+  uint32_t hc0 = 0u;
+  const uint32_t hstep = hover ? 2u * kHS : (uint32_t)a.span;
+  auto count_chunk = [&](uint32_t c0) __attribute__((always_inline)) {
+    __syncthreads();  // the chunk before was read
+    for (uint32_t e = 4u * (uint32_t)tid; e < kHS; e += 4u * (uint32_t)kThreads)
+      *reinterpret_cast<uint4 *>(L.hent + e) = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    for (int i0 = h0 + tid; i0 < h1; i0 += 8 * kThreads) {
+      uint32_t hb8[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) hb8[j] = i0 + j * kThreads < h1 ? hid[i0 + j * kThreads] : kEmpty;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t off = hb8[j] - (uint32_t)lo;
+        if (off < (uint32_t)nids && off - c0 < 2u * kHS)
+          atomicAdd(&L.hent[(off - c0) >> 1], 1u << (16u * (off & 1u)));
+      }
+    }
+    __syncthreads();
+    hc0 = c0;
+  };
+  auto occurrences = [&](uint32_t off) __attribute__((always_inline)) -> uint32_t {
+    if (hover) return (L.hent[(off - hc0) >> 1] >> (16u * (off & 1u))) & 0xFFFFu;
+    return hcount(off);
+  };
+  if (has_hist && hover) {
+    // (the allowed members' bitmap is still in LDS after one pass; parts of
+    // several take the exact selection)
+    const bool lists = s_qover == 0u && npass == 1;
+    __syncthreads();
+    if (tid == 0) {
+      s_nx = 0u;
+      s_nmw = 0u;  // member records the cut may have written are rewritten
+    }
+    __syncthreads();
+    for (uint32_t c0 = 0u; lists && c0 < (uint32_t)nids; c0 += hstep) {
+      if (hover) count_chunk(c0);
+      // thread t: the members among 2^sh2 ids from c0 + 2^sh2 t on, the next
+      // one's value loading while one is penalized
+      const uint32_t len = min((uint32_t)nids - c0, hstep);
+      const uint32_t sh2 = 32u - (uint32_t)__builtin_clz((len - 1u) / (uint32_t)kThreads | 1u);
+      const uint32_t o0 = c0 + ((uint32_t)tid << sh2);
+      uint32_t rest = o0 < c0 + len ? (L.hmem[o0 >> 5] >> (o0 & 31u)) & (~0u >> (32u - (1u << sh2))) : 0u;
+      auto next = [&]() __attribute__((always_inline)) {
+        return rest ? lrow[(uint32_t)lo + o0 + (uint32_t)__builtin_ctz(rest)] : qnan();
+      };
+      float xn = next();
+      while (rest) {
+        const uint32_t o = o0 + (uint32_t)__builtin_ctz(rest);
+        float x = xn;
+        rest &= rest - 1u;
+        xn = next();
+        if (kSoftcap && softcap > 0.0f) x = softcap_f32(x, softcap);
+        const double pen = penalize((double)x, occurrences(o), p);
+        if (pen >= (double)tff) {  // NaN never passes
+          const uint32_t d = atomicAdd(&s_nx, 1u);
+          if (d < (uint32_t)kXCap) {
+            L.x_val[d] = pen;
+            L.x_id[d] = (uint32_t)lo + o;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    nx = nxm = s_nx;
+    exact = !lists || nx > (uint32_t)kXCap || nw[0] + nw[1] + nw[2] + nw[3] + nx > (uint32_t)kListCap;
+    xw = (uint32_t)tid < nx && !exact;
+    if (xw) {
+      xv = L.x_val[tid];
+      xid = L.x_id[tid];
+    }
+  }
+  if (exact) {
     // more values at or above the bound than the lists hold (ties): the
     // part's exact top k by a radix select over (value, id) keys, every
     // value read again from memory
-    const int rounds = (nids + kThreads - 1) / kThreads;
     auto for_elems = [&](auto f) {
-      for (int i = 0; i < rounds; ++i) {
-        const uint32_t off = (uint32_t)(i * kThreads + tid);
-        const uint32_t id = (uint32_t)lo + off;
-        bool ok = off < (uint32_t)nids;
-        uint32_t cnt = 0u;
-        float x = 0.0f;
-        double val = 0.0;
-        if (ok) {
-          const uint32_t mw = kMask ? mrow[id >> 5] | mall : ~0u;
-          x = lrow[id];
-          cnt = has_hist ? hcount(id) : 0u;
-          ok = !kMask || ((mw >> (id & 31u)) & 1u);
-          if (kSoftcap && softcap > 0.0f) x = softcap_f32(x, softcap);
-          ok = ok && x == x;
-          val = cnt ? penalize((double)x, cnt, p) : (double)x;
-          ok = ok && val == val;
+      for (uint32_t c0 = 0u; c0 < (uint32_t)nids; c0 += hstep) {
+        if (hover) count_chunk(c0);
+        const uint32_t end = min((uint32_t)nids, c0 + hstep);
+        for (uint32_t o = c0; o < end; o += (uint32_t)kThreads) {
+          const uint32_t off = o + (uint32_t)tid, id = (uint32_t)lo + off;
+          bool ok = off < end;
+          uint32_t cnt = 0u;
+          float x = 0.0f;
+          double val = 0.0;
+          if (ok) {
+            const uint32_t mw = kMask ? mrow[id >> 5] | mall : ~0u;
+            x = lrow[id];
+            cnt = has_hist ? occurrences(off) : 0u;
+            ok = !kMask || ((mw >> (id & 31u)) & 1u);
+            if (kSoftcap && softcap > 0.0f) x = softcap_f32(x, softcap);
+            ok = ok && x == x;
+            val = cnt ? penalize((double)x, cnt, p) : (double)x;
+            ok = ok && val == val;
+          }
+          f(key96(val, id), ok, val, id | (cnt ? kXMem : 0u), x, cnt);
         }
-        f(key96(val, id), ok, val, id | (cnt ? kXMem : 0u), x, cnt);
       }
     };
     uint32_t nval = 0u;

@@ -598,3 +598,99 @@ def test_element_types_are_checked_each_time(sampler):
             sampler.sample_into(x, ids, mask=mask.to(torch.int64), params=Params())
         with pytest.raises(ValueError, match="uniforms must hold"):
             sampler.sample_into(x, ids, uniforms=torch.zeros(2, device="cuda"), params=Params(temperature=1.0))
+
+
+# ------------------------------------------- many history ids in one part --
+
+_DISTINCT = [
+    # vocab, rows, ids of row 0's history in [lo, hi), each `reps` times, other rows' ids each.  The hash holds
+    # 1,024 ids of a part (2,048 of bucketed histories, 1,024 ids a row on average), one slot per id in parts of
+    # no more ids; past that the ids are counted 2,048 (4,096) at a time
+    (1000, 2, 0, 1000, 1, 20),                # a part of 1,000 ids, all of them members
+    (1024, 1, 3, 1024, 1, 0),
+    (1000, 1, 0, 900, 3, 0),                  # bucketed
+    (262_144, 16, 24_576, 25_476, 1, 100),    # 900 ids of an 8,192-id part: probing
+    (262_144, 16, 24_570, 26_100, 2, 100),    # 1,524 of them: counted in four chunks
+    (262_144, 16, 24_576, 32_768, 1, 100),    # all 8,192
+    (262_144, 2, 100_000, 101_900, 2, 1500),  # bucketed: 1,900 ids over two parts
+    (262_144, 2, 98_304, 106_496, 7, 1500),   # bucketed: all 8,192 ids of a part, in two chunks
+    (600_000, 1, 20_000, 21_000, 1, 0),       # parts of two passes
+    (600_000, 1, 17_000, 31_000, 1, 0),       # bucketed, two passes, four chunks
+    (600_000, 2, 17_000, 19_000, 1, 3),
+]
+
+
+@pytest.mark.parametrize("vocab,rows,lo,hi,reps,others", _DISTINCT)
+@pytest.mark.parametrize("kind", ["lower", "raise", "greedy", "softcap"])
+def test_many_distinct_history_ids_in_a_part(sampler, vocab, rows, lo, hi, reps, others, kind):
+    rng = np.random.default_rng(vocab + lo + hi + reps)
+    x = (rng.standard_normal((rows, vocab)) * 2.0).astype(np.float32)
+    ids = np.concatenate([np.arange(lo, hi)] * reps + [np.repeat(rng.integers(lo, hi, 40), 3)])
+    x[0, rng.integers(lo, hi, 60)] += np.float32(6.0)  # members among the row's best
+    x[0, rng.integers(0, vocab, 60)] += np.float32(5.0)
+    hist = [rng.permutation(ids)] + [rng.integers(0, vocab, others) for _ in range(rows - 1)]
+    hi_, ho = W._csr(hist)
+    p = {"lower": Params(temperature=0.9, top_k=60, top_p=0.95, repetition_penalty=1.2, presence_penalty=0.3,
+                         frequency_penalty=0.2),
+         "raise": Params(temperature=1.0, top_k=128, top_p=1.0, repetition_penalty=0.9, frequency_penalty=0.1),
+         "greedy": Params(temperature=0.0, repetition_penalty=1.3, frequency_penalty=0.5),
+         "softcap": Params(temperature=1.0, top_k=50, top_p=0.9, repetition_penalty=1.1, presence_penalty=0.5,
+                           softcap=30.0)}[kind]
+    mask = W.random_mask(rng, rows, vocab, 0.6, 0.9) if kind in ("raise", "softcap") else None
+    b = W.Batch("distinct", x, p, mask=mask, hist_ids=hi_, hist_offsets=ho, uniforms=rng.random(rows))
+    print(f"[gpu] {len(hist[0])} history ids in [{lo}, {hi}) of {vocab}, rows={rows} {kind}", flush=True)
+    check(sampler, b, label=f"distinct {kind}")
+
+
+@pytest.mark.parametrize("vocab,off", [(262_144, 0), (262_144, 8191), (1000, 999)])
+def test_largest_count_of_one_history_id(sampler, vocab, off):
+    # SAS_MAX_HISTORY occurrences of one id, at a part's first and last id
+    rng = np.random.default_rng(vocab + off)
+    x = rng.standard_normal((1, vocab)).astype(np.float32)
+    x[0, off] = np.float32(9.0)
+    x[0, 500] = np.float32(8.0)
+    hi, ho = W._csr([np.full(65_535, off)])
+    for f in (1e-5, 2e-5):  # 9 - 65,535 f: above 8, below
+        b = W.Batch("count", x, Params(temperature=1.0, top_k=20, top_p=1.0, frequency_penalty=f), hist_ids=hi,
+                    hist_offsets=ho, uniforms=np.array([0.3]))
+        print(f"[gpu] 65,535 occurrences of id {off}, frequency {f}", flush=True)
+        g, _ = check(sampler, b, label="count")
+        assert (g["cand_ids"][0, 0] == off) == (f == 1e-5)
+
+
+def _us_per_call(fn, n=10):
+    import torch
+    best = 1e9
+    for _ in range(3):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        fn()
+        torch.cuda.synchronize()
+        e0.record()
+        for _ in range(n):
+            fn()
+        e1.record()
+        torch.cuda.synchronize()
+        best = min(best, e0.elapsed_time(e1) / n * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("vocab,lo,hi,n", [(1000, 0, 1000, 1000), (1000, 0, 1000, 8000), (262_144, 8192, 16_384, 8000),
+                                           (262_144, 8192, 16_384, 65_535)])
+def test_distinct_history_ids_cost_no_scan_each(sampler, vocab, lo, hi, n):
+    # counting a part's history takes a few reads of it however many distinct
+    # ids it holds, never a read per id: within 40 times a call with 64 ids
+    # (a scan per id took 200 to 8,000 times)
+    import torch
+    rng = np.random.default_rng(n)
+    x = to_dev((rng.standard_normal((1, vocab)) * 3.0).astype(np.float32))
+    out = torch.empty(1, dtype=torch.int32, device="cuda")
+    us = []
+    for m in (64, n):
+        ids = to_dev(rng.integers(lo, hi, m).astype(np.int32))
+        offs = to_dev(np.array([0, m], np.int32))
+        p = Params(temperature=0.7, top_k=40, top_p=0.95, repetition_penalty=1.1, frequency_penalty=0.2)
+        us.append(_us_per_call(lambda: sampler.sample_into(x, out, hist_ids=ids, hist_offsets=offs, params=p,
+                                                           uniforms=torch.full((1,), 0.5, dtype=torch.float64,
+                                                                               device="cuda"))))
+    print(f"[gpu] vocab {vocab}: 64 ids {us[0]:.1f} us, {n} ids in [{lo}, {hi}) {us[1]:.1f} us", flush=True)
+    assert us[1] < 40 * us[0]
