@@ -694,3 +694,25 @@ def test_distinct_history_ids_cost_no_scan_each(sampler, vocab, lo, hi, n):
                                                                                device="cuda"))))
     print(f"[gpu] vocab {vocab}: 64 ids {us[0]:.1f} us, {n} ids in [{lo}, {hi}) {us[1]:.1f} us", flush=True)
     assert us[1] < 40 * us[0]
+
+
+@pytest.mark.parametrize("kind", ["lower", "raise", "greedy", "softcap"])
+@pytest.mark.parametrize("vocab,lo,hi,n", [(8192, 0, 8192, 4000), (1000, 0, 1000, 600), (262_144, 8192, 16_384, 700),
+                                           (262_144, 8000, 9216, 700), (5003, 0, 5003, 3000)])
+def test_many_members_in_a_part_stay_on_the_lists(sampler, vocab, lo, hi, n, kind):
+    # more allowed history members in a part than its exact list holds (256),
+    # few of them at the bound: no exact selection (no SAS_FLAG_SLOW_SELECT)
+    rng = np.random.default_rng(vocab + lo + n)
+    rows = 8
+    x = (rng.standard_normal((rows, vocab)) * 2.0).astype(np.float32)
+    x[0, rng.integers(lo, hi, 5)] += np.float32(6.0)
+    hi_, ho = W._csr([rng.integers(lo, hi, n)] + [rng.integers(0, vocab, 100) for _ in range(rows - 1)])
+    p = {"lower": Params(temperature=0.9, top_k=30, top_p=0.95, repetition_penalty=1.2, presence_penalty=0.3),
+         "raise": Params(temperature=1.0, top_k=20, top_p=1.0, repetition_penalty=0.9, frequency_penalty=0.1),
+         "greedy": Params(temperature=0.0, repetition_penalty=1.3, frequency_penalty=0.5),
+         "softcap": Params(temperature=1.0, top_k=25, top_p=0.9, presence_penalty=0.5, softcap=30.0)}[kind]
+    mask = W.random_mask(rng, rows, vocab, 0.9, 0.99) if kind == "softcap" else None
+    b = W.Batch("many_members", x, p, mask=mask, hist_ids=hi_, hist_offsets=ho, uniforms=rng.random(rows))
+    print(f"[gpu] {n} history ids in [{lo}, {hi}) of {vocab} {kind}", flush=True)
+    g, _ = check(sampler, b, label=f"many members {kind}")
+    assert not np.any(g["flags"] & FLAG_SLOW_SELECT), g["flags"]
