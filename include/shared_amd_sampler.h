@@ -243,9 +243,10 @@ typedef struct sas_reserve_desc {
                                 sas_spec_step (their draft rows are counted in) */
   int32_t vocab;             /* 1..SAS_MAX_VOCAB, the vocabulary of every call below */
   int64_t hist_ids;          /* the most history ids of one call (hist_count, or
-                                rows * ring_len for sas_sample_step, seqs * ring_len
-                                for sas_spec_step): long histories
-                                (>= 1,024 ids per row) are bucketed in scratch */
+                                rows * ring_len for the step calls, seqs * ring_len
+                                for sas_spec_step): long histories (>= 1,024 ids per
+                                row, >= 4,096 behind the LM head) are bucketed in
+                                scratch */
   int32_t lm_head_rows;      /* 0, or the rows of sas_lm_head_sample (<= SAS_LMH_MAX_ROWS;
                                 vocab <= SAS_LMH_MAX_VOCAB) */
   int32_t verify_seqs;       /* 0, or the sequences of sas_verify ... */

@@ -220,10 +220,9 @@ struct SpecDraw {
 };
 
 // sas_sample, sas_sample_step (st) and the sampling of sas_spec_exact (sp):
-// one checked descriptor's launches.  bucket: long histories may be
-// bucketed first (not behind the LM head, whose scratch holds no buckets).
+// one checked descriptor's launches.  head: the logits are the LM head's.
 int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char *who, void *stream,
-              const SpecDraw *sp = nullptr, bool bucket = true) {
+              const SpecDraw *sp = nullptr, bool head = false) {
   if (int rc = set_device(s)) return rc;
   // at least two blocks per CU: small batches take shorter parts
   int parts = 0, span = 0;
@@ -272,7 +271,13 @@ int sample_on(sas_sampler *s, const sas_rows *r, const sas_step *st, const char 
   const int hrows = sp && sp->group > 1 ? r->rows / sp->group : r->rows;
   const bool ring = a.ring != nullptr;
   const int64_t hist_ids = ring ? (int64_t)hrows * a.ring_len : (r->hist_ids ? r->hist_count : 0);
-  if (bucket && hist_ids >= sas::kBucketMinIds * hrows && hist_ids > 0) {
+  a.long_hist = hist_ids >= sas::kBucketMinIds * hrows && hist_ids > 0;
+  bool bucket = a.long_hist;
+  if (head)
+    // (without buckets where a capture has no scratch for them)
+    bucket = parts > 1 && hist_ids >= sas::kHeadBucketMinIds * hrows && hist_ids > 0 &&
+             (hb_bytes(hist_ids, hrows, parts) <= s->hb_cap || !capturing(stream));
+  if (bucket) {
     const size_t ids_bytes = ((size_t)hist_ids * 4 + 255) & ~size_t(255);
     if (int rc = grow(s, &s->hb, &s->hb_cap, hb_bytes(hist_ids, hrows, parts), stream, who)) return rc;
     a.hb_ids = reinterpret_cast<uint32_t *>(s->hb);
@@ -373,7 +378,7 @@ int lm_head_on(sas_sampler *s, const sas_lm_head *h, const sas_rows *r, const sa
   sas_rows lr = *r;
   lr.logits = a.logits;
   lr.logits_stride = a.logits_stride;
-  return sample_on(s, &lr, st, who, stream, nullptr, false);
+  return sample_on(s, &lr, st, who, stream, nullptr, true);
 }
 
 }  // namespace
@@ -463,8 +468,9 @@ int sas_reserve_for(sas_sampler *s, const sas_reserve_desc *d) {
   // the most parts any batch of <= rows rows may pick (a single row)
   int parts = 0, span = 0;
   sas::choose_parts(1, d->vocab, 2 * s->cus, &parts, &span);
-  if (d->hist_ids >= sas::kBucketMinIds && d->rows > 0)
-    if (int rc = grow(s, &s->hb, &s->hb_cap, hb_bytes(d->hist_ids, d->rows, parts), nullptr, who)) return rc;
+  const int hrows = std::max(d->rows, d->lm_head_rows);
+  if (d->hist_ids >= sas::kBucketMinIds && hrows > 0)
+    if (int rc = grow(s, &s->hb, &s->hb_cap, hb_bytes(d->hist_ids, hrows, parts), nullptr, who)) return rc;
   if (d->verify_seqs > 0)
     if (int rc = grow(s, &s->vscratch, &s->vscratch_cap,
                       sas::verify_scratch_bytes(d->verify_seqs, d->verify_draft_len, d->vocab), nullptr, who))

@@ -17,7 +17,7 @@
 //      the part reach it, so no value below it is in the row's top k;
 //   4. values at or above the bound go to per-wave LDS lists (one ballot per
 //      value slot); the part's history ids are handled one by one with their
-//      exact penalized double values (with long, bucketed histories and
+//      exact penalized double values (with long histories and
 //      penalties that only lower values, members ride in the lists with
 //      their raw values and only those reaching the bound are penalized);
 //   5. the lists are written as records to the part's own slots: plain
@@ -889,7 +889,7 @@ static_assert(kXCap >= SAS_MAX_TOP_K, "an exact part selection fits the exact li
 constexpr uint32_t kXMem = 0x80000000u;
 
 // The hash of a part's history ids: entries of 16 bits each, the id's place
-// in the part and its occurrences, 0 where empty.  Bucketed (long) histories
+// in the part and its occurrences, 0 where empty.  Long histories
 // take twice the slots (six blocks per CU still fit).  Where an id finds no
 // slot the members are counted again, in chunks (count_chunk): a few reads of
 // the history, not one per id.  One row of 1,000 ids with 1,000 uniform
@@ -918,8 +918,8 @@ struct PartLds {
 // the same XCD (rows stay on one XCD), so from L2.
 __device__ __forceinline__ void put_rec(uint64_t *p, uint64_t v) { *p = v; }
 
-// kList: the history is bucketed (long histories, kHist only): members may
-// ride in the lists (see `lower`).
+// kList: long histories (kHist only): members may ride in the lists (see
+// `lower`).
 template <bool kMask, bool kHist, bool kSoftcap, bool kList>
 __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6) void sample_parts_kernel(const SampleArgs a) {
   __shared__ __attribute__((aligned(16))) PartLds<kList> L;
@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
     return 0u;
   };
   // ---- passes: values, the bound, the lists ---------------------------------
-  // Long (bucketed) histories, whose members are many, with penalties that
+  // Long histories, whose members are many, with penalties that
   // only lower values (repetition >= 1, frequency >= 0, presence >= 0;
   // rounding keeps this): a member whose raw value is below the bound stays
   // below it, so members ride in the lists with their raw values and only
@@ -1756,9 +1756,9 @@ __global__ __launch_bounds__(kBucketThreads) void hist_bucket_kernel(const Sampl
 
 template <bool kMask, bool kHist, bool kSoftcap>
 static void launch_kernel(const SampleArgs &a, hipStream_t stream) {
-  // the list mode pays only with the many members of long (bucketed)
-  // histories; short ones keep collecting members in the slot loop
-  if (kHist && a.hb_offs)
+  // the list mode pays only with the many members of long histories; short
+  // ones keep collecting members in the slot loop
+  if (kHist && a.long_hist)
     hipLaunchKernelGGL((sample_parts_kernel<kMask, kHist, kSoftcap, kHist>), dim3((unsigned)(a.rows * a.parts)),
                        dim3(kThreads), 0, stream, a);
   else

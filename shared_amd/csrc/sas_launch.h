@@ -86,6 +86,7 @@ struct SampleArgs {
   // Null: every part scans its row's whole history.
   uint32_t *hb_ids;
   int32_t *hb_offs;
+  bool long_hist;  // kBucketMinIds or more ids per row: the parts kernel's list variants
   int32_t vocab;
   int32_t rows;
   int32_t parts;   // blocks per row
@@ -121,7 +122,11 @@ hipError_t launch_spec_cascade(const uint32_t *picks, const uint32_t *drafts, co
 // Histories of at least this many ids per row on average are bucketed by
 // part first (one more launch): each part then reads its own ids only.
 constexpr int64_t kBucketMinIds = 1024;
-
+// Behind the LM head (1 to 4 rows, one block to bucket each) from this many
+// on: a call of one row of 32,000 ids x 1,024 takes 27.7 us with 2,048 ids
+// scanned by every part, 30 bucketed; of 262,144 ids with 4,096 102.8, 99.0,
+// with 65,535 1,109, 153.
+constexpr int64_t kHeadBucketMinIds = 4096;
 
 // Scratch bytes of the records and part counts for a batch shape.
 size_t sample_rec_bytes(int rows, int parts);

@@ -22,6 +22,17 @@ def to_dev(a, dtype=None):
     return t.cuda()
 
 
+def graph_nodes(g) -> int:
+    """Nodes of a captured torch.cuda.CUDAGraph(keep_graph=True)."""
+    import ctypes
+    from shared_amd import _capi
+    hip = _capi.load()  # its HIP runtime's symbols are found behind it
+    n = ctypes.c_size_t(0)
+    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    assert hip.hipGraphGetNodes(g.raw_cuda_graph(), None, ctypes.byref(n)) == 0
+    return n.value
+
+
 def run_gpu(s: Sampler, b, *, logits_dev=None, row_params=None, full=True):
     import torch
     lg = logits_dev if logits_dev is not None else to_dev(b.logits)

@@ -9,7 +9,7 @@ between the replays; a graph over persistent buffers follows their contents."""
 import numpy as np
 import pytest
 
-from gpu_helpers import to_dev
+from gpu_helpers import graph_nodes, to_dev
 from shared_amd import DecodeState, Params, Sampler
 from shared_amd import workloads as W
 from shared_amd._capi import MAX_TOP_K
@@ -307,3 +307,38 @@ def test_head_with_caller_logits_needs_no_logits_scratch():
                 err = str(ex)
         torch.cuda.synchronize()
         assert err is not None and "being captured" in err, err
+
+
+@pytest.mark.parametrize("hist,reserved,nodes", [(2000, True, 3), (5000, True, 4), (5000, False, 3), (65_535, True, 4)])
+def test_head_over_long_histories_in_a_graph(hist, reserved, nodes):
+    """Behind the LM head, histories of 4,096 ids a row or more are bucketed
+    (head, buckets, parts, merge) when the handle's scratch holds them; a
+    capture on a handle without that scratch scans them in the parts.  Ids,
+    candidates and flags are the same, none from an exact selection."""
+    import torch
+    from shared_amd._capi import FLAG_SLOW_SELECT
+    b = W.lmh(rows=2, vocab=40_000, dim=256, seed=45, hist=hist, mask=False)
+    print(f"[gpu] graph: lm head, {hist} history ids a row, reserved {reserved}", flush=True)
+    hid, wt = to_dev(b.hidden), to_dev(b.weight_bits.view(np.int16))
+    out = {**_outs(b.rows), "flags": torch.empty(b.rows, dtype=torch.int32, device="cuda")}
+    kw = dict(hist_ids=to_dev(b.hist_ids, torch.int32), hist_offsets=to_dev(b.hist_offsets),
+              uniforms=to_dev(b.uniforms), params=b.params, **{f"out_{k}": v for k, v in out.items() if k != "ids"})
+    with Sampler(0) as e:
+        e.lm_head_sample_into(hid, wt, out["ids"], **kw)
+        torch.cuda.synchronize()
+        want = _host(out)
+    if hist < 65_535:  # (there nearly every id of a part is a member)
+        assert not np.any(want["flags"] & FLAG_SLOW_SELECT)
+    with Sampler(0) as s:
+        s.reserve(0, b.vocab, hist_ids=b.rows * hist if reserved else 0, lm_head_rows=b.rows)
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            s.lm_head_sample_into(hid, wt, out["ids"], **kw)
+        assert graph_nodes(g) == nodes
+        g.instantiate()
+        for rep in range(REPLAYS):
+            _scrub(out)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            _equal(_host(out), want, f"long history replay {rep}")

@@ -365,3 +365,18 @@ def test_quantized_operand_of_special_hidden_states(sampler, fmt):
     assert np.array_equal(np.isnan(g["logits"]), np.isnan(lo))
     fine = ~np.isnan(lo)
     assert np.array_equal(g["logits"][fine].view(np.uint32), lo[fine].view(np.uint32))
+
+
+@pytest.mark.parametrize("vocab,lo,hi,hist", [(1000, 0, 1000, 1000), (1000, 0, 1000, 5000), (30_000, 0, 30_000, 2000),
+                                              (100_000, 4096, 12_288, 1500), (100_000, 4096, 12_288, 3500),
+                                              (100_000, 0, 100_000, 12_000), (100_000, 4096, 12_288, 65_535)])
+@pytest.mark.parametrize("raises", [False, True])
+def test_long_histories_behind_the_head(sampler, vocab, lo, hi, hist, raises):
+    # histories of 1,024 ids a row and more take the list variants, of 4,096
+    # and more the buckets; more distinct ids in a part than its hash holds
+    rng = np.random.default_rng(vocab + lo + hist)
+    b = W.lmh(rows=2, vocab=vocab, dim=256, seed=hist + lo, hist=0, mask=False)
+    b.hist_ids, b.hist_offsets = W._csr([rng.integers(lo, hi, hist), rng.integers(0, vocab, hist)])
+    b.params = Params(temperature=0.9, top_k=30, top_p=0.95, repetition_penalty=0.9 if raises else 1.2,
+                      presence_penalty=0.0 if raises else 0.5, frequency_penalty=0.1, softcap=30.0 if raises else 0.0)
+    check(sampler, b, f"history {hist} in [{lo}, {hi})")

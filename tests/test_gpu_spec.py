@@ -9,7 +9,7 @@ import oracle as O
 from shared_amd import Params, SasError
 from shared_amd import workloads as W
 from shared_amd.sampler import pack_params, row_hints
-from gpu_helpers import oracle_chain
+from gpu_helpers import graph_nodes, oracle_chain
 
 pytestmark = pytest.mark.gpu
 
@@ -248,17 +248,6 @@ def test_draft_rows_ride_with_the_verify_rows(sampler, seqs, vocab, L, softcap):
         p.softcap = softcap
     print(f"[gpu] spec riding drafts seqs={seqs} vocab={vocab} L={L} softcap={softcap}", flush=True)
     check(run_spec(sampler, c), O.spec_exact(c), f"riding {seqs}x{vocab} L{L}")
-
-
-def graph_nodes(g) -> int:
-    """Nodes of a captured torch.cuda.CUDAGraph(keep_graph=True)."""
-    import ctypes
-    from shared_amd import _capi
-    hip = _capi.load()  # its HIP runtime's symbols are found behind it
-    n = ctypes.c_size_t(0)
-    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
-    assert hip.hipGraphGetNodes(g.raw_cuda_graph(), None, ctypes.byref(n)) == 0
-    return n.value
 
 
 @pytest.mark.parametrize("rows,nodes", [(3, 3), (2, 5)])
