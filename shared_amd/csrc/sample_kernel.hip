@@ -1766,27 +1766,26 @@ static void launch_kernel(const SampleArgs &a, hipStream_t stream) {
                        dim3(kThreads), 0, stream, a);
 }
 
-template <int kT>
-static void launch_merge_threads(const SampleArgs &a, int slots, hipStream_t stream) {
-  const dim3 grid((unsigned)a.rows), block(kT);
-  constexpr int kMost = kT == 1024 ? 8 : kMRMax;
-  if (slots <= 4) hipLaunchKernelGGL((sample_merge_kernel<4, kT>), grid, block, 0, stream, a);
-  else if (slots <= 8) hipLaunchKernelGGL((sample_merge_kernel<8, kT>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((sample_merge_kernel<kMost, kT>), grid, block, 0, stream, a);
+template <int kMR, int kT>
+static void launch_merge_as(const SampleArgs &a, hipStream_t stream) {
+  hipLaunchKernelGGL((sample_merge_kernel<kMR, kT>), dim3((unsigned)a.rows), dim3(kT), 0, stream, a);
 }
 
 // Threads and record slots per thread of the merge.  A part emits about k to
 // 2 k records (its bound certifies k of its own values; ties and the bound's
 // slack add more), so slots for 2 k + 8 records of every part hold nearly
-// all of them.  Per-row parameters are unknown here: the largest k.
+// all of them (up to 16 a thread, 8 of 1,024 threads; the rest are read
+// again).  Per-row parameters are unknown here: the largest k.
 //
-// A row's records are one block's work: past 2,048 of them 512 threads read
-// and rank them faster (8 rows of 262,144 ids in 64 parts, k = 64: 14.5 ->
-// 9.1 us; 128 rows, k = 50: 8.1 -> 8.0), past 10,240 (40 parts or more) 1,024
-// threads (9 rows in 52 parts, k = 128: 53.8, 18.0 with 512, 15.2); below,
-// the barriers of more waves cost more than they save (64 rows of 151,936
-// ids, k = 40: 6.6 us with 256 threads, 7.2 with 512, 9.8 with 1,024; a call
-// of 8 rows of 262,144 ids in 32 parts, k = 128: 19.5 us with 512, 20.4 with
+// A row's records are one block's work.  Past 2,048 of them 512 threads read
+// and rank them faster (calls, 256 -> 512 threads: 8 rows of 262,144 ids in
+// 32 parts at k = 40 12.2 -> 11.7 us, k = 64 13.6 -> 13.3, k = 128 22.0 ->
+// 15.1; 64 rows of 151,936 ids at k = 50 16.9 -> 16.7), past 10,240 (39 parts
+// or more: over 311,296 ids) 1,024 threads (512 -> 1,024: 8 rows of 400,000
+// ids in 49 parts at k = 100 16.9 -> 17.7, 110 18.4 -> 17.6, 128 20.9 -> 19.3; 4 rows of
+// 524,288 ids in 64 parts at k = 128 28.6 -> 23.1).  Below the borders the
+// barriers of more waves cost more than they save (64 rows of 151,936 ids,
+// k = 40, this kernel: 6.6 us with 256 threads, 7.2 with 512, 9.8 with
 // 1,024).
 static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
   if (a.parts < 1 || a.parts > kMaxParts) return hipErrorInvalidValue;  // the merge's count table
@@ -1794,9 +1793,17 @@ static hipError_t launch_merge(const SampleArgs &a, hipStream_t stream) {
   const int k = greedy ? 1 : a.row_params ? SAS_MAX_TOP_K : std::min(std::max(a.params.top_k, 1), SAS_MAX_TOP_K);
   const int per = 2 * k + 8, records = per * a.parts;
   auto slots = [&](int threads) { return (per + threads / a.parts - 1) / (threads / a.parts); };
-  if (greedy || records <= 2048) launch_merge_threads<256>(a, slots(256), stream);
-  else if (records <= 10240) launch_merge_threads<512>(a, slots(512), stream);
-  else launch_merge_threads<1024>(a, slots(1024), stream);
+  if (greedy || records <= 2048) {
+    const int n = slots(256);
+    if (n <= 4) launch_merge_as<4, 256>(a, stream);
+    else if (n <= 8) launch_merge_as<8, 256>(a, stream);
+    else launch_merge_as<kMRMax, 256>(a, stream);
+  } else if (records <= 10240) {  // more than 4 slots
+    if (slots(512) <= 8) launch_merge_as<8, 512>(a, stream);
+    else launch_merge_as<kMRMax, 512>(a, stream);
+  } else {  // more than 8
+    launch_merge_as<8, 1024>(a, stream);
+  }
   return hipGetLastError();
 }
 

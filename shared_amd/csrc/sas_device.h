@@ -240,17 +240,6 @@ constexpr int kDppQuad1032 = 0xB1, kDppQuad2301 = 0x4E, kDppRowHalfMirror = 0x14
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
 constexpr int kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
 
-// Inclusive prefix sum over the wave: Hillis-Steele within each row of 16
-// lanes, then the rows' totals broadcast forward.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-  x += dpp0<kDppRowShr1>(x);
-  x += dpp0<kDppRowShr2>(x);
-  x += dpp0<kDppRowShr4>(x);
-  x += dpp0<kDppRowShr8>(x);
-  x += dpp0<kDppRowBcast15, 0xA>(x);
-  x += dpp0<kDppRowBcast31, 0xC>(x);
-  return x;
-}
 
 // Wave-wide reductions: pairs, quads, eights and rows of 16 by DPP, then the
 // four rows' results (wave-uniform).
@@ -273,12 +262,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
 // exact search.
 __device__ __forceinline__ uint32_t wave_rank_key(uint32_t u, int j) {
   return j == 1 ? wave_max_u32(u) : wave_jth_largest_key16(u, j);
-}
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-  return wave_reduce(x, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
-}
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {
-  return wave_reduce(x, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 // Lane i's double on every lane (i wave-uniform).

@@ -94,8 +94,9 @@ struct SampleArgs {
 };
 
 // Parts per row and ids per part for a batch shape: spans of one pass
-// (fewer, larger parts) unless the grid would hold fewer than
-// `min_blocks` blocks (then at most 32); at most kMaxParts parts per row.
+// (fewer, larger parts) unless the grid would hold fewer than `min_blocks`
+// blocks (then shorter parts, at most 32: up to 262,144 ids); at most
+// kMaxParts parts per row.
 void choose_parts(int rows, int vocab, int min_blocks, int *parts, int *span);
 // Launches the sampling kernel on `stream`.  softcap: some row may have a
 // softcap (row_params, or params.softcap > 0).
