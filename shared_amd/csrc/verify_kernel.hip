@@ -103,8 +103,9 @@ struct ExpTab {
 __device__ __forceinline__ f64x2 exp_tab_entry() { return kExp2Tab[threadIdx.x & (kExpTab - 1)]; }
 
 // e^x for sums of many weights, x <= 0, where the order of the additions
-// already differs from a sequential loop: within 0.82 ulp of the exact value
-// (rms 0.296 ulp, over 8 million x in [-700, 0] against 113-bit arithmetic;
+// already differs from a sequential loop (the table-driven method of P. T. P.
+// Tang, ACM TOMS 15, 1989): within 0.82 ulp of the exact value (rms 0.296
+// ulp, over 8 million x in [-700, 0] against 113-bit arithmetic;
 // a degree-13 series without a table: 0.86 and 0.302), with no division.
 // x = k ln2 / 64 + r, |r| <= ln2 / 128 (k by adding 1.5 * 2^52, ln2 / 64
 // split in two parts, the high one with 21 zero bits), e^r - 1 by its Taylor
