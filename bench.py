@@ -54,7 +54,7 @@ WORKLOAD_DOC = {
             "row, then C3P's mask, penalties and top-k 50 / top-p 0.9",
     "LMQ3": "as LMQ1 with the three rows of a speculative verify round over the same head",
 }
-CPU_THREADS = 16  # the GPU box's CPU share for one GPU (its nproc may show more)
+CPU_THREADS = 16  # a host CPU share for one GPU (nproc may show more)
 
 
 def parse_args():
@@ -558,7 +558,7 @@ def main() -> int:
     args = parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
-        print(f"bench.py: this build measures one GPU only (asked for --gpus {args.gpus}, WORLD_SIZE {world}); "
+        print(f"bench.py measures one GPU only (asked for --gpus {args.gpus}, WORLD_SIZE {world}); "
               "rows shard across GPUs with no exchange, so run one process per GPU.", file=sys.stderr)
         return 2
     if args.calibrate_copy_mb > 0:

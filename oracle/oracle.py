@@ -1,7 +1,7 @@
-"""ctypes wrapper of the C oracle and a driver for the Node restatement.
+"""ctypes wrapper of the C oracle and a runner of the Node restatement.
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and
-bench.py's cpu_baseline leg, as the checker.  Never on the product path.
+bench.py's cpu_baseline leg, as the oracle.  Never on the product path.
 """
 from __future__ import annotations
 

@@ -2,7 +2,7 @@
 /*
  * sample_js.js - Node restatement of the reference sampling path.
  *
- * TEST INFRASTRUCTURE ONLY: the parity checker and the CPU baseline that
+ * TEST INFRASTRUCTURE ONLY: the oracle and the CPU baseline that
  * bench.py times on the host cores.  The product never loads it.
  *
  * It keeps the reference's two-stage CPU structure:

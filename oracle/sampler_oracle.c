@@ -54,7 +54,7 @@
  *                      a planted block, ties to even, numpy's float16.
  *   orc_lm_head_q_logits  the GGUF heads (ggml/kernels.js:64-80 dequant
  *                      formulas; the Q8_1 GEMV terms of ggml/q8.js:202-240)
- *                      in this build's order.  Pinned by closed forms: a
+ *                      in the library's order.  Pinned by closed forms: a
  *                      block's weights recovered through one-hot hiddens
  *                      (scale 127 exactness), every block term against the
  *                      reference's per-element dequantization formula in

@@ -2,7 +2,7 @@
  * sampler_oracle.h - CPU oracle for the logit-processing / sampling path.
  *
  * TEST INFRASTRUCTURE ONLY.  Only tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py may load this code, and only as the checker.
+ * cpu_baseline leg of bench.py may load this code, and only as the oracle.
  * The product library (shared_amd/) never links or calls it.
  *
  * The oracle restates, in plain C with IEEE doubles and no FMA contraction,

@@ -23,7 +23,7 @@
 // the same block left CUs idle below 131,072 ids, and folding their records
 // took a launch of its own.  A whole call before -> now: Q4_0 32,000 x
 // 4,096, one row, 91.7 -> 31.2 us; Q6_K 248,320 x 2,560, three rows, 129.2
-// -> 117.9 us; bf16 262,144 x 2,560, one row, 217.1 -> 215.0 us, 6.7 TB/s
+// -> 117.9 us; bf16 262,144 x 2,560, one row, 217.1 -> 208.8 us, 7.0 TB/s
 // in this kernel.)
 #include "sas_device.h"
 #include "sas_launch.h"

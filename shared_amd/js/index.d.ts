@@ -1,13 +1,13 @@
 // Types of the Node host API (index.js).  The mask and parameter shapes are
 // the reference's: TokenMask (lib/webgpu-llm/tool-constraint.ts:39-42) and
-// SampleParams (lib/webgpu-llm/model.d.ts:4-16), with the build's
+// SampleParams (lib/webgpu-llm/model.d.ts:4-16), with the library's
 // additional penalties.
 
 export type TokenMask =
   | { kind: "all" }
   | { kind: "allow"; tokenIds: Uint32Array }
   | { kind: "deny"; tokenIds: Uint32Array }
-  /** This build's extension: packed words (ceil(vocab / 32), bit id & 31 of word id >> 5 = allowed). */
+  /** An extension: packed words (ceil(vocab / 32), bit id & 31 of word id >> 5 = allowed). */
   | { kind: "words"; words: Uint32Array };
 
 /** Packed-bitmask producer for grammar code; results are immutable words arrays. */

@@ -37,7 +37,7 @@ check('mask uploads once per distinct immutable mask', function () {
   sas.updateTokenMaskState(state, { kind: 'deny', tokenIds: tokenIds });
   assert.strictEqual(state.uploads.length, 1);
   // a new array with the same ids: the reference uploads it again; its words
-  // equal the ones on the device, so this build does not
+  // equal the ones on the device, so the library does not
   sas.updateTokenMaskState(state, { kind: 'deny', tokenIds: Uint32Array.of(1, 2, 3) });
   assert.strictEqual(state.uploads.length, 1);
   sas.updateTokenMaskState(state, { kind: 'deny', tokenIds: Uint32Array.of(1, 2, 4) });
