@@ -678,8 +678,8 @@ def _us_per_call(fn, n=10):
                                            (262_144, 8192, 16_384, 65_535)])
 def test_distinct_history_ids_cost_no_scan_each(sampler, vocab, lo, hi, n):
     # counting a part's history takes a few reads of it however many distinct
-    # ids it holds, never a read per id: within 40 times a call with 64 ids
-    # (a scan per id took 200 to 8,000 times)
+    # ids it holds, never a read per id: within 100 times a call with 64 ids
+    # (2 to 35 times; a scan per id took 150 to 14,000 times)
     import torch
     rng = np.random.default_rng(n)
     x = to_dev((rng.standard_normal((1, vocab)) * 3.0).astype(np.float32))
@@ -693,7 +693,7 @@ def test_distinct_history_ids_cost_no_scan_each(sampler, vocab, lo, hi, n):
                                                            uniforms=torch.full((1,), 0.5, dtype=torch.float64,
                                                                                device="cuda"))))
     print(f"[gpu] vocab {vocab}: 64 ids {us[0]:.1f} us, {n} ids in [{lo}, {hi}) {us[1]:.1f} us", flush=True)
-    assert us[1] < 40 * us[0]
+    assert us[1] < 100 * us[0]
 
 
 @pytest.mark.parametrize("kind", ["lower", "raise", "greedy", "softcap"])
