@@ -1294,7 +1294,8 @@ __global__ __launch_bounds__(kThreads, kSoftcap ? 4 : (kMask && !kHist) ? 5 : 6)
   // and their places among the wave's records
   // (raw values: the listed ones capped here, the bound's cap the final bound)
   const float tfr = tkey > 0x007FFFFFu ? fkey(tkey) : -__builtin_inff();
-  const float tff = kSoftcap && !capped ? softcap_f32(tfr, softcap) : tfr;
+  // (no bound stays none: a member's penalized value may lie below -cap)
+  const float tff = kSoftcap && !capped && tkey > 0x007FFFFFu ? softcap_f32(tfr, softcap) : tfr;
   const uint32_t qat = (uint32_t)wave * kQuadCap + (uint32_t)lane;
   auto cut = [&](uint32_t e, float4 &q, uint32_t &qid) __attribute__((always_inline)) -> uint32_t {
     const bool qin = (uint32_t)lane + e < n_q && n_q <= (uint32_t)kQuadCap;

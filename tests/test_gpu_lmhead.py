@@ -90,8 +90,8 @@ def test_long_history_and_unmasked(sampler):
 
 def test_members_fill_a_part(sampler):
     # every id of the first 1,024 is in the history with identity penalties:
-    # parts 0 and 1 hold only members (more than a part's member slots), so
-    # their exact slow selection runs
+    # the first part (1,024 ids) holds only members, more than its member
+    # slots, so its exact slow selection runs
     b = W.lmh(rows=1, vocab=4096, dim=256, seed=12, hist=0, mask=False)
     ids = np.arange(1024, dtype=np.uint32)
     b.hist_ids, b.hist_offsets = ids, np.array([0, ids.size], np.int32)
@@ -380,3 +380,22 @@ def test_long_histories_behind_the_head(sampler, vocab, lo, hi, hist, raises):
     b.params = Params(temperature=0.9, top_k=30, top_p=0.95, repetition_penalty=0.9 if raises else 1.2,
                       presence_penalty=0.0 if raises else 0.5, frequency_penalty=0.1, softcap=30.0 if raises else 0.0)
     check(sampler, b, f"history {hist} in [{lo}, {hi})")
+
+
+@pytest.mark.parametrize("temperature", [0.0, 1.0])
+def test_members_below_minus_softcap_behind_the_head(sampler, temperature):
+    # the only allowed ids are history members whose frequency penalties take
+    # them below -softcap: they are still the row's candidates
+    rng = np.random.default_rng(77)
+    b = W.lmh(rows=3, vocab=5000, dim=256, seed=78, hist=0)
+    bits = np.zeros((3, 5000), bool)
+    hist = []
+    for r in range(3):
+        allowed = rng.choice(5000, 1 + 2 * r, replace=False)
+        bits[r, allowed] = True
+        hist.append(np.repeat(allowed, 25 + 5 * r))
+    b.mask = W.pack_bits(bits)
+    b.hist_ids, b.hist_offsets = W._csr(hist)
+    b.params = Params(temperature=temperature, top_k=20, top_p=0.95, frequency_penalty=2.0, softcap=30.0)
+    g, _ = check(sampler, b, f"members below -softcap T={temperature}")
+    assert (g["ids"] != NO_TOKEN).all()

@@ -716,3 +716,32 @@ def test_many_members_in_a_part_stay_on_the_lists(sampler, vocab, lo, hi, n, kin
     print(f"[gpu] {n} history ids in [{lo}, {hi}) of {vocab} {kind}", flush=True)
     g, _ = check(sampler, b, label=f"many members {kind}")
     assert not np.any(g["flags"] & FLAG_SLOW_SELECT), g["flags"]
+
+
+def below_the_cap(rng, rows, vocab):
+    """Rows whose allowed ids are all history members, many of them repeated
+    until the frequency penalty takes them below -softcap."""
+    bits = np.zeros((rows, vocab), bool)
+    hist = []
+    for r in range(rows):
+        allowed = rng.choice(vocab, int(rng.integers(1, 6)), replace=False)
+        bits[r, allowed] = True
+        hist.append(np.concatenate([np.repeat(allowed, rng.integers(20, 60, allowed.size)), rng.integers(0, vocab, 30)]))
+    hi, ho = W._csr(hist)
+    return W.pack_bits(bits), hi, ho
+
+
+@pytest.mark.parametrize("vocab", [7, 1000, 50_000])
+@pytest.mark.parametrize("temperature", [0.0, 1.0])
+def test_members_below_minus_softcap(sampler, vocab, temperature):
+    # a softcap row's part without a plain value has no bound: its members
+    # count whatever their penalized values
+    rng = np.random.default_rng(vocab)
+    rows = 6
+    x = (rng.standard_normal((rows, vocab)) * 5.0).astype(np.float32)
+    mask, hi, ho = below_the_cap(rng, rows, vocab)
+    p = Params(temperature=temperature, top_k=20, top_p=0.95, frequency_penalty=2.0, presence_penalty=0.5, softcap=30.0)
+    b = W.Batch("below_cap", x, p, mask=mask, hist_ids=hi, hist_offsets=ho, uniforms=rng.random(rows))
+    print(f"[gpu] members below -softcap vocab={vocab} T={temperature}", flush=True)
+    g, _ = check(sampler, b, label="below_cap")
+    assert (g["ids"] != NO_TOKEN).all()
